@@ -91,7 +91,7 @@ typedef struct {
     int nOut;               /* nsampBuf - maxshift - remainingSamples */
     float mstartdm;         /* dmLow / tsamp (float) */
     float mdmstep;          /* dmStep / tsamp (float) */
-    int tileDM, tileT;      /* DM x time tile chosen for this plan */
+    int tileDM, tileT;      /* DM x time tile chosen for this plan (see ppl_dedisp_plan_create) */
     int chanBlock;          /* channels staged per block (0: as many as fit in LDS) */
     int readBytes;          /* LDS read width per lane of the chosen kernel: 4 or 16 */
     long long fusedDelayDiffs; /* delay entries that would differ were the trial value
@@ -103,15 +103,19 @@ typedef struct {
 /* DedispersionModule::resize (src/lib/src/DedispersionModule.cpp:109-190):
  * builds the FP32 delay table on the host from the FP64 shift table exactly
  * as the reference (:152-162, DedispersionKernel.cu:29,36), uploads it and
- * picks the tile shape: for FP32 input the ring kernel at 32 trials x 512
- * samples where a tile's delay spread fits its staged row, else (and for
- * f16 and u8) the one-word kernel at 32 (or fewer) trials x 512.  Fails with PPL_E_CONFIG when nsampBuf <= maxshift
+ * picks the kernel: for FP32 and FP16 rows of whole 16-byte pieces the
+ * register-window kernel, in a shape that its sizes call for, and beside it a
+ * tile for the others (input that is not 16-byte aligned, a tile set later):
+ * for FP32 the ring kernel at 32 trials x 512 samples where a tile's delay
+ * spread fits its staged row, else (and for f16 and u8) the one-word kernel at
+ * 32 (or fewer) trials x 512.  ppl_dedisp_info reports that tile.  Fails with PPL_E_CONFIG when nsampBuf <= maxshift
  * (the module's throw at :175-178), when dmStep < 0 (delays would decrease
  * with the trial index) or when a delayed read would leave the channel row. */
 int ppl_dedisp_plan_create(ppl_dedisp_plan** plan, const ppl_dedisp_config* cfg);
 int ppl_dedisp_plan_destroy(ppl_dedisp_plan* plan);
 int ppl_dedisp_plan_info(const ppl_dedisp_plan* plan, ppl_dedisp_info* info);
-/* Override the DM x time tile (the autotuner's hook); 0 keeps the default. */
+/* Override the DM x time tile (the autotuner's hook); 0 keeps the default.  A
+ * plan whose tile was set runs that tile and not the window kernel. */
 int ppl_dedisp_set_tile(ppl_dedisp_plan* plan, int tileDM, int tileT);
 /* Same with the number of channels staged per LDS block (0: as many as fit). */
 int ppl_dedisp_set_shape(ppl_dedisp_plan* plan, int tileDM, int tileT, int chanBlock);
@@ -121,9 +125,12 @@ int ppl_dedisp_set_shape(ppl_dedisp_plan* plan, int tileDM, int tileT, int chanB
  * 32, byte count of the input a multiple of 4; tileT 256 or 512).  All give
  * the same sums bit for bit. */
 int ppl_dedisp_set_kernel(ppl_dedisp_plan* plan, int tileDM, int tileT, int chanBlock, int readBytes);
-/* Autotuner: times every instantiated DM x time tile, channel block and read width on
- * the given buffers (reps launches each, HIP events on the stream), keeps the
- * fastest for the plan and returns its time per launch in *best_ms. */
+/* Takes a set or tuned tile back: the plan runs as one just created. */
+int ppl_dedisp_clear_tile(ppl_dedisp_plan* plan);
+/* Autotuner: times the kernel the plan's sizes call for and every instantiated
+ * DM x time tile, channel block and read width on the given buffers (reps
+ * launches each, HIP events on the stream), keeps the fastest for the plan
+ * (the first as no tile set) and returns its time per launch in *best_ms. */
 int ppl_dedisp_autotune(ppl_dedisp_plan* plan, const void* d_in, void* d_out, int reps, void* stream,
                         float* best_ms);
 /* Copy the int32 delay table [tdms][nChan] to host memory (for checks). */
@@ -140,10 +147,11 @@ int ppl_dedisperse(const ppl_dedisp_plan* plan, const void* d_in, void* d_out, v
  * reference dedisperses one beam per GPU job, DedispersionModule.cpp:263-297).
  * Each job is a plan with its own input buffer and output; plans may differ
  * in channels, buffer length, DM count and range, but share the dtype.  All
- * jobs run under one DM x time tile, channel block and read width (tileDM =
- * tileT = 0: the first plan's; when that is a ring tile another job's delay
- * spread does not fit, the same tile with one-word reads), each with its own
- * LDS row length.  Results equal n separate ppl_dedisperse calls, bit for
+ * jobs run under one DM x time tile, channel block and read width, each with
+ * its own LDS row length; with tileDM = tileT = 0 under the first plan's tile
+ * if one was set (when that is a ring tile another job's delay spread does
+ * not fit, the same tile with one-word reads), else each under the kernel its
+ * sizes call for, one launch per kernel.  Results equal n separate ppl_dedisperse calls, bit for
  * bit. */
 typedef struct {
     const ppl_dedisp_plan* plan;
@@ -154,7 +162,9 @@ enum { PPL_DEDISP_MAX_JOBS = 48 };
 int ppl_dedisperse_batch(const ppl_dedisp_job* jobs, int n, int tileDM, int tileT, int chanBlock,
                          int readBytes, void* stream);
 /* Autotuner for a batch: times every instantiated tile, channel block and
- * read width that fits every job (reps launches each) and returns the fastest. */
+ * read width that fits every job (reps launches each) and, where the first
+ * plan has no tile set, no tile at all; returns the fastest (tileDM = tileT =
+ * 0 for the last). */
 int ppl_dedisp_autotune_batch(const ppl_dedisp_job* jobs, int n, int reps, void* stream, int* tileDM,
                               int* tileT, int* chanBlock, int* readBytes, float* best_ms);
 

@@ -94,6 +94,7 @@ SIGNATURES = {
     "ppl_dedisp_set_tile": (i, [vp, i, i]),
     "ppl_dedisp_set_shape": (i, [vp, i, i, i]),
     "ppl_dedisp_set_kernel": (i, [vp, i, i, i, i]),
+    "ppl_dedisp_clear_tile": (i, [vp]),
     "ppl_dedisp_autotune": (i, [vp, vp, vp, i, vp, vp]),
     "ppl_dedisp_delays": (i, [vp, vp]),
     "ppl_dedisperse": (i, [vp, vp, vp, vp]),
@@ -226,6 +227,7 @@ class DedispPlan:
         self.maxshift, self.rem, self.nout = info.maxshift, info.remainingSamples, info.nOut
         self.mstartdm, self.mdmstep = info.mstartdm, info.mdmstep
         self.tile = (info.tileDM, info.tileT, info.chanBlock, info.readBytes)
+        self.own_tile = False  # no tile set: launches run the kernel the sizes call for
         # delays that a contracted (fused multiply-add) trial value would change
         self.fused_delay_diffs = info.fusedDelayDiffs
 
@@ -243,14 +245,23 @@ class DedispPlan:
         """Tile (DM trials x samples), channels staged per block (0: as many
         as fit) and LDS read width per lane (4, or 16 for FP32 input)."""
         check(lib().ppl_dedisp_set_kernel(self.h, tile_dm, tile_t, chan_block, read_bytes))
+        self.own_tile = self.own_tile or (tile_dm, tile_t) != (0, 0)
+        self._refresh()
+
+    def clear_tile(self):
+        """Back to no tile set: launches run the kernel the sizes call for."""
+        check(lib().ppl_dedisp_clear_tile(self.h))
+        self.own_tile = False
         self._refresh()
 
     def autotune(self, d_in, d_out, reps=2, stream=None):
-        """Time every tile shape / channel block on these buffers and keep the fastest."""
+        """Time the kernel the sizes call for and every tile shape / channel
+        block on these buffers and keep the fastest."""
         best = C.c_float(0)
         check(lib().ppl_dedisp_autotune(self.h, _ptr(d_in), _ptr(d_out), reps, _stream(stream),
                                         C.byref(best)))
         self._refresh()
+        self.own_tile = self.tile[2] != 0  # every tile it tries has a channel block
         return best.value
 
     def delays(self):
@@ -321,7 +332,7 @@ def dedisperse_batch(plans, d_ins, d_outs=None, tile=(0, 0, 0, 4), stream=None):
             raise PPLError("tile must be a (tileDM, tileT, chanBlock[, readBytes]) tuple or 'own'")
         groups = {}
         for k, p in enumerate(plans):
-            groups.setdefault(tuple(p.tile), []).append(k)
+            groups.setdefault(tuple(p.tile) if p.own_tile else (0, 0, 0, 4), []).append(k)
         for t, ks in groups.items():
             dedisperse_batch([plans[k] for k in ks], [d_ins[k] for k in ks], [d_outs[k] for k in ks], tile=t,
                              stream=stream)
@@ -1231,7 +1242,7 @@ class MultiBeam:
             return ms
         # per-beam tiles (each tuned alone), kept only if the grouped launches
         # beat the single batch tile on the whole batch
-        old = [p.tile for p in self.plans]
+        old = [p.tile if p.own_tile else None for p in self.plans]
         for p, x, o in zip(self.plans, ins, self.outs):
             t, _ = autotune_batch([p], [x], [o], reps=reps, candidates=candidates)
             p.set_tile(*t)
@@ -1247,7 +1258,10 @@ class MultiBeam:
             self.tile = "own"
             return own_ms
         for p, t in zip(self.plans, old):
-            p.set_tile(*t)
+            if t is None:
+                p.clear_tile()
+            else:
+                p.set_tile(*t)
         return ms
 
     def chunk_lengths(self, b, n_spec):

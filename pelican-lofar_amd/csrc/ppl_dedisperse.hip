@@ -15,6 +15,8 @@
 // bound by LDS bandwidth (one 4-byte read per add); FP16 and u8 inputs halve
 // and quarter the bytes per add.
 #include "ppl_internal.h"
+#include "ppl_dedisp_jobs.h"
+#include "ppl_dedisp_window.h"
 
 #include <algorithm>
 #include <cmath>
@@ -39,6 +41,12 @@ struct ppl_dedisp_plan {
     // offsets of each trial's reads, then per tile and channel the first
     // trial's delay
     int32_t* d_ring[3] = {nullptr, nullptr, nullptr};  // ring tables for DM tiles of 16, 32, 64
+    // the window kernel's table (ppl_dedisp_window.h; null: the plan does not
+    // take that kernel), shape (an index of kWinShapes) and staging
+    int4* d_win = nullptr;
+    int winShape = 0, winStaging = 0;
+    bool ownTile = false;  // a tile was set (by the caller or the autotuner)
+    int defNd = 8, defNt = 8, defRw = 4;  // the tile the plan started with
     // u8 series, built on first use: per trial dm, the number of channels
     // whose delay is k, for k = 0 .. maxdelay(dm): lenTab[lenOff[dm] + k];
     // lenOff[tdms] is the table's length
@@ -68,43 +76,11 @@ template <> struct Acc<uint8_t> { using type = int32_t; };
 // whole time tiles (x, x+8, ...), and the DM tiles of one time tile follow
 // one another on it, so their overlapping delayed input rows are fetched
 // from HBM about once per time tile instead of once per XCD.
-constexpr int kXcds = 8;
 __device__ __forceinline__ void tile_of(int bid, int nDMTiles, int& tTile, int& dmTile)
 {
     const int xcd = bid % kXcds, k = bid / kXcds;
     tTile = (k / nDMTiles) * kXcds + xcd;
     dmTile = k % nDMTiles;
-}
-
-// One beam's part of a launch.  A launch covers several beams (jobs): job k
-// owns workgroups [blockStart, blockStart + nDMTiles*nTTilesPad), a multiple
-// of 8, so a job's own XCD-major tile order is kept.  The table travels in
-// the kernel arguments; a workgroup finds its job with a uniform scan.
-constexpr int kMaxDDJobs = PPL_DEDISP_MAX_JOBS;
-struct DDJob {
-    const void* in;
-    void* out;
-    const int32_t* delayT;
-    int nChan, nsamp, tdms, tdmsPad, nOut;
-    int rowUnits;   // LDS row length: elements (f32) or dwords per copy (f16, u8)
-    int CB;         // channels per staged block
-    int nDMTiles;
-    int blockStart;
-    int pad_;
-};
-struct DDBatch {
-    DDJob job[kMaxDDJobs];
-    int n;
-    float one;  // 1.0f, kept opaque to the compiler (f16 kernel)
-};
-
-__device__ __forceinline__ const DDJob& find_job(const DDBatch& B, int& local)
-{
-    int jb = 0;
-    for (int k = 1; k < B.n; ++k)
-        if ((int)blockIdx.x >= B.job[k].blockStart) jb = k;
-    local = (int)blockIdx.x - B.job[jb].blockStart;
-    return B.job[jb];
 }
 
 template <typename Tin, int ND, int NT>
@@ -279,18 +255,6 @@ constexpr int ring_quads_of_tile(int TD) { return ring_quads(TD == 64 ? 8 : 4); 
 #define PPL_RING_DEPTH 3
 #endif
 
-// s_waitcnt bounding only the vector memory counter (gfx9 encoding:
-// vmcnt[3:0] in bits 3:0, vmcnt[5:4] in bits 15:14; expcnt and lgkmcnt at
-// their maxima, i.e. not waited for).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt()
-{
-    static_assert(N >= 0 && N < 64, "vmcnt out of range");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-__device__ __forceinline__ void bare_barrier() { asm volatile("s_barrier" ::: "memory"); }
-
 // Twelve LDS-DMA dword loads of consecutive 64-dword rows: row k from
 // global address g + 256k to LDS address lds + 256k (+ 4 * lane each).  The
 // address is the uniform row start g in scalar registers plus the lane's
@@ -345,12 +309,6 @@ __device__ __forceinline__ void dma_rows8(const float* g, uint32_t laneBytes, ui
                  : "=&s"(saved)
                  : "v"(laneBytes), "s"(g), "s"(lds)
                  : "memory");
-}
-
-// LDS address (byte offset in the workgroup's LDS) of a __shared__ pointer.
-__device__ __forceinline__ uint32_t lds_addr(const void* p)
-{
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
 // Reads of the staged rows in inline assembly, each block waiting for its
@@ -1387,7 +1345,7 @@ int make_job(const ppl_dedisp_plan* p, const Shape& s, const void* in, void* out
     J.CB = CB;
     J.nDMTiles = (J.tdms + TD - 1) / TD;
     J.blockStart = 0;
-    J.pad_ = 0;
+    J.nTiles = 0;
     *ldsBytes = s.rw == 16 ? 0 : (size_t)CB * perChannel;  // the 16-byte kernel's LDS is static
     return PPL_OK;
 }
@@ -1534,6 +1492,113 @@ int run_jobs(const ppl_dedisp_job* jobs, int n, const Shape& s, hipStream_t st)
     return PPL_E_ARG;
 }
 
+// The window kernel's shapes, the widest of a type first, with the stagings
+// that hold a tile of theirs.
+struct WinEntry {
+    int E, TT;
+    void (*table)(const int32_t*, int, int, int, int, int, int4*);
+    void (*kernel[kWinStagings])(DDBatch);
+};
+template <class S, int G>
+constexpr void (*win_kernel())(DDBatch)
+{
+    if constexpr (16 / S::E * (S::TT + 2 * S::E) <= win_stage_bytes(G))
+        return dedisperse_window_kernel<S, G>;
+    else
+        return nullptr;
+}
+template <class S>
+constexpr WinEntry win_entry()
+{
+    return {S::E, S::TT, win_table_kernel<S>,
+            {win_kernel<S, kWinSplit1>(), win_kernel<S, kWinSplit2>(), win_kernel<S, kWinSplit4>(),
+             win_kernel<S, kWinWhole2>(), win_kernel<S, kWinWhole4>()}};
+}
+const WinEntry kWinShapes[] = {win_entry<WinF32>(), win_entry<WinF32Short>(), win_entry<WinF32Small>(),
+                               win_entry<WinF16>(), win_entry<WinF16Small>()};
+
+// Jobs whose plan has no tile set run the kernel that its sizes call for: the
+// window kernel where the plan has its table and the input is 16-byte aligned
+// (rows then start on 16 bytes: the table is only built for such row
+// lengths), else the plan's first tile.  One launch per kernel and tile.
+bool takes_window(const ppl_dedisp_job& jb)
+{
+    return (reinterpret_cast<uintptr_t>(jb.d_in) & 15) == 0 && jb.plan->d_win;
+}
+
+int run_window(const ppl_dedisp_job* const* jobs, int n, hipStream_t st)
+{
+    const WinEntry& W = kWinShapes[jobs[0]->plan->winShape];
+    DDBatch B{};
+    B.n = n;
+    long blocks = 0;
+    for (int k = 0; k < n; ++k) {
+        const ppl_dedisp_plan* p = jobs[k]->plan;
+        DDJob& J = B.job[k];
+        J.in = jobs[k]->d_in;
+        J.out = jobs[k]->d_out;
+        J.delayT = reinterpret_cast<const int32_t*>(p->d_win);
+        J.nChan = (int)p->cfg.nChan;
+        J.nsamp = (int)p->cfg.nsampBuf;
+        J.tdms = (int)p->cfg.tdms;
+        J.nOut = p->nOut;
+        J.nDMTiles = (J.tdms + kWinTD - 1) / kWinTD;
+        const long tiles = (long)J.nDMTiles * ((J.nOut + W.TT - 1) / W.TT);
+        PPL_CHECK_ARG(blocks + tiles + kXcds < (1L << 31), "grid too large");
+        J.nTiles = (int)tiles;
+        J.blockStart = (int)blocks;
+        blocks += (tiles + kXcds - 1) / kXcds * kXcds;
+    }
+    hipLaunchKernelGGL(W.kernel[jobs[0]->plan->winStaging], dim3((unsigned)blocks), dim3(64 * kWinWaves), 0, st, B);
+    PPL_LAUNCHED();
+    return PPL_OK;
+}
+
+int run_default(const ppl_dedisp_job* jobs, int n, hipStream_t st)
+{
+    PPL_CHECK_ARG(n >= 1 && n <= kMaxDDJobs, "%d dedispersion jobs (1..%d)", n, kMaxDDJobs);
+    for (int k = 0; k < n; ++k) {
+        PPL_CHECK_ARG(jobs[k].plan && jobs[k].d_in && jobs[k].d_out, "job %d: null argument", k);
+        PPL_CHECK_ARG(jobs[k].plan->cfg.dtype == jobs[0].plan->cfg.dtype, "job %d: dtype differs from job 0", k);
+    }
+    // longest workgroups first (see run_jobs)
+    int order[kMaxDDJobs];
+    for (int k = 0; k < n; ++k) order[k] = k;
+    std::stable_sort(order, order + n, [&](int a, int b) {
+        return jobs[a].plan->cfg.nChan > jobs[b].plan->cfg.nChan;
+    });
+    bool done[kMaxDDJobs] = {};
+    for (int k = 0; k < n; ++k) {
+        const ppl_dedisp_plan* p = jobs[order[k]].plan;
+        if (done[order[k]] || !takes_window(jobs[order[k]])) continue;
+        const ppl_dedisp_job* same[kMaxDDJobs];
+        int m = 0;
+        for (int i = k; i < n; ++i) {
+            const ppl_dedisp_job& jb = jobs[order[i]];
+            if (!takes_window(jb) || jb.plan->winShape != p->winShape || jb.plan->winStaging != p->winStaging) continue;
+            done[order[i]] = true;
+            same[m++] = &jb;
+        }
+        const int rc = run_window(same, m, st);
+        if (rc != PPL_OK) return rc;
+    }
+    for (int k = 0; k < n; ++k) {
+        if (done[k]) continue;
+        const ppl_dedisp_plan* p = jobs[k].plan;
+        ppl_dedisp_job same[kMaxDDJobs];
+        int m = 0;
+        for (int i = k; i < n; ++i) {
+            const ppl_dedisp_plan* q = jobs[i].plan;
+            if (done[i] || q->defNd != p->defNd || q->defNt != p->defNt || q->defRw != p->defRw) continue;
+            done[i] = true;
+            same[m++] = jobs[i];
+        }
+        const int rc = run_jobs(same, m, Shape{p->defNd, p->defNt, 0, p->defRw}, st);
+        if (rc != PPL_OK) return rc;
+    }
+    return PPL_OK;
+}
+
 const Shape kShapes[] = {{8, 8, 0}, {8, 4, 0}, {4, 8, 0}, {4, 4, 0}, {2, 8, 0}, {16, 4, 0}, {16, 2, 0},
                          {4, 8, 0, 16}, {8, 8, 0, 16}, {4, 4, 0, 16}, {8, 4, 0, 16}, {16, 8, 0, 16},
                          {16, 4, 0, 16}};
@@ -1579,6 +1644,53 @@ int upload_delays(ppl_dedisp_plan* p)
     PPL_HIP(hipMemcpy(p->d_delayT, t.data(), t.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     p->tdmsPad = pad;
     for (int k = 0; k < 4; ++k) p->spanTD[k] = tile_span(p->delays, tdms, nChan, 8 << k);
+    return PPL_OK;
+}
+
+// The window kernel's shape for a plan's sizes, or -1: rows of whole 16-byte
+// pieces, and 32-trial tiles whose delay spread one of its stages holds.  The
+// widest shape whose tiles keep the 256 CUs busy, else the shortest: one tile
+// a CU is enough for FP32 (517 trials x 31584 samples x 8704 channels, 425
+// wide tiles: 4.9 ms against 6.3 at 12 samples a lane; 512 x 17248 x 496, 224
+// wide tiles: 0.45 against 0.40), half that for FP16, whose only shorter shape
+// is a third as long (the same sizes, 192 wide tiles: 0.38 ms against 0.54).
+int window_shape(int dtype, int tdms, int nOut, int span, int* staging)
+{
+    if (dtype == PPL_U8) return -1;
+    const int E = dtype == PPL_F32 ? 4 : 8;
+    const long dmTiles = (tdms + kWinTD - 1) / kWinTD;
+    int pick = -1;
+    for (int k = 0; k < (int)(sizeof(kWinShapes) / sizeof(kWinShapes[0])); ++k) {
+        const WinEntry& W = kWinShapes[k];
+        if (W.E != E) continue;
+        const int g = win_staging(E, W.TT, span);
+        if (g < 0) continue;
+        pick = k;
+        *staging = g;
+        if (dmTiles * ((nOut + W.TT - 1) / W.TT) >= (E == 4 ? 256 : 128)) break;
+    }
+    return pick;
+}
+
+// The window kernel's table, built on the device from the plan's delays.
+int window_table(ppl_dedisp_plan* p)
+{
+    const int nChan = (int)p->cfg.nChan, nsamp = (int)p->cfg.nsampBuf, elem = elem_bytes(p->cfg.dtype);
+    int staging = 0;
+    const int shape = window_shape(p->cfg.dtype, (int)p->cfg.tdms, p->nOut, span_of(p, kWinTD), &staging);
+    if (shape < 0 || (long)nsamp * elem % 16 != 0 || (long)p->nOut * elem % 16 != 0 ||
+        (long)nChan * nsamp >= (1L << 31))
+        return PPL_OK;
+    const int nDMTiles = ((int)p->cfg.tdms + kWinTD - 1) / kWinTD;
+    const size_t bytes = win_table_bytes(nDMTiles, nChan);
+    PPL_HIP(hipMalloc(&p->d_win, bytes));
+    const size_t n = bytes / sizeof(int4);
+    hipLaunchKernelGGL(kWinShapes[shape].table, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, nullptr, p->d_delayT,
+                       nChan, nsamp, p->tdmsPad, nDMTiles, win_whole(staging), p->d_win);
+    PPL_LAUNCHED();
+    PPL_HIP(hipStreamSynchronize(nullptr));  // the plan may be used on any stream
+    p->winShape = shape;
+    p->winStaging = staging;
     return PPL_OK;
 }
 
@@ -1673,9 +1785,13 @@ extern "C" int ppl_dedisp_plan_create(ppl_dedisp_plan** plan, const ppl_dedisp_c
             p->rw = 16;
         }
     }
+    p->defNd = p->nd;
+    p->defNt = p->nt;
+    p->defRw = p->rw;
     int rc = upload_delays(p);
+    if (rc == PPL_OK) rc = window_table(p);
     if (rc != PPL_OK) {
-        delete p;
+        ppl_dedisp_plan_destroy(p);
         return rc;
     }
     *plan = p;
@@ -1688,6 +1804,7 @@ extern "C" int ppl_dedisp_plan_destroy(ppl_dedisp_plan* plan)
     if (plan->d_delayT) (void)hipFree(plan->d_delayT);
     for (int32_t* t : plan->d_ring)
         if (t) (void)hipFree(t);
+    if (plan->d_win) (void)hipFree(plan->d_win);
     if (plan->d_lenOff) (void)hipFree(plan->d_lenOff);
     if (plan->d_lenTab) (void)hipFree(plan->d_lenTab);
     delete plan;
@@ -1747,48 +1864,91 @@ extern "C" int ppl_dedisp_set_kernel(ppl_dedisp_plan* p, int tileDM, int tileT, 
     p->nt = s.nt;
     p->cb = s.cb;
     p->rw = s.rw;
+    p->ownTile = true;
     return PPL_OK;
 }
 
-extern "C" int ppl_dedisp_autotune(ppl_dedisp_plan* p, const void* d_in, void* d_out, int reps, void* stream,
-                                   float* best_ms)
+extern "C" int ppl_dedisp_clear_tile(ppl_dedisp_plan* p)
 {
-    PPL_CHECK_ARG(p && d_in && d_out, "null argument");
+    PPL_CHECK_ARG(p, "null plan");
+    p->nd = p->defNd;
+    p->nt = p->defNt;
+    p->rw = p->defRw;
+    p->cb = 0;
+    p->ownTile = false;
+    return PPL_OK;
+}
+
+namespace {
+// Time per launch of `run` over reps launches after an untimed one, HIP
+// events on the stream; PPL_OK and *ms = infinity where it refuses the shape.
+template <typename F>
+int time_launch(F run, int reps, hipEvent_t e0, hipEvent_t e1, hipStream_t st, float* ms)
+{
+    *ms = INFINITY;
+    if (run() != PPL_OK) return PPL_OK;
+    PPL_HIP(hipEventRecord(e0, st));
+    for (int r = 0; r < reps; ++r)
+        if (run() != PPL_OK) break;
+    PPL_HIP(hipEventRecord(e1, st));
+    PPL_HIP(hipEventSynchronize(e1));
+    PPL_HIP(hipEventElapsedTime(ms, e0, e1));
+    *ms /= reps;
+    return PPL_OK;
+}
+
+// Fastest of the kernels that the jobs' sizes call for (best->nd = 0; left
+// out unless `free`) and every instantiated tile and channel block that fits
+// all the jobs.
+int fastest_shape(const ppl_dedisp_job* jobs, int n, bool free, int reps, hipStream_t st, Shape* best,
+                  float* best_ms)
+{
     if (reps < 1) reps = 1;
-    hipStream_t st = stream_of(stream);
     hipEvent_t e0, e1;
     PPL_HIP(hipEventCreate(&e0));
     PPL_HIP(hipEventCreate(&e1));
+    *best = Shape{0, 0, 0};
+    *best_ms = INFINITY;
+    int rc = free ? time_launch([&] { return run_default(jobs, n, st); }, reps, e0, e1, st, best_ms) : PPL_OK;
     const int cbs[] = {1, 2, 4, 8, 16};
-    float best = 1e30f;
-    Shape bestShape{p->nd, p->nt, p->cb, p->rw};
     for (const Shape& base : kShapes) {
-        if (!shape_for(base, p->cfg.dtype)) continue;
+        if (!shape_for(base, jobs[0].plan->cfg.dtype)) continue;
         for (int cb : cbs) {
             const Shape s{base.nd, base.nt, cb, base.rw};
-            DDJob J{};
-            size_t lds = 0;
-            if (make_job(p, s, d_in, d_out, J, &lds) != PPL_OK || J.CB < cb) continue;
-            const ppl_dedisp_job job{p, d_in, d_out};
-            if (run_jobs(&job, 1, s, st) != PPL_OK) continue;  // warm
-            PPL_HIP(hipEventRecord(e0, st));
-            for (int r = 0; r < reps; ++r)
-                if (run_jobs(&job, 1, s, st) != PPL_OK) break;
-            PPL_HIP(hipEventRecord(e1, st));
-            PPL_HIP(hipEventSynchronize(e1));
+            bool fits = rc == PPL_OK;
+            for (int k = 0; k < n && fits; ++k) {
+                DDJob J{};
+                size_t lds = 0;
+                fits = jobs[k].plan && make_job(jobs[k].plan, s, jobs[k].d_in, jobs[k].d_out, J, &lds) == PPL_OK &&
+                       J.CB >= cb;
+            }
+            if (!fits) continue;
             float ms = 0.0f;
-            PPL_HIP(hipEventElapsedTime(&ms, e0, e1));
-            ms /= reps;
-            if (ms < best) {
-                best = ms;
-                bestShape = s;
+            rc = time_launch([&] { return run_jobs(jobs, n, s, st); }, reps, e0, e1, st, &ms);
+            if (ms < *best_ms) {
+                *best_ms = ms;
+                *best = s;
             }
         }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    if (best_ms) *best_ms = best;
-    return ppl_dedisp_set_kernel(p, 4 * bestShape.nd, 64 * bestShape.nt, bestShape.cb, bestShape.rw);
+    return rc;
+}
+}  // namespace
+
+extern "C" int ppl_dedisp_autotune(ppl_dedisp_plan* p, const void* d_in, void* d_out, int reps, void* stream,
+                                   float* best_ms)
+{
+    PPL_CHECK_ARG(p && d_in && d_out, "null argument");
+    const ppl_dedisp_job job{p, d_in, d_out};
+    Shape best;
+    float ms = 0.0f;
+    const int rc = fastest_shape(&job, 1, true, reps, stream_of(stream), &best, &ms);
+    if (rc != PPL_OK) return rc;
+    if (best_ms) *best_ms = ms;
+    if (best.nd == 0) return ppl_dedisp_clear_tile(p);
+    return ppl_dedisp_set_kernel(p, 4 * best.nd, 64 * best.nt, best.cb, best.rw);
 }
 
 extern "C" int ppl_dedisp_delays(const ppl_dedisp_plan* p, int32_t* host_out)
@@ -1802,6 +1962,7 @@ extern "C" int ppl_dedisperse(const ppl_dedisp_plan* p, const void* d_in, void* 
 {
     PPL_CHECK_ARG(p && d_in && d_out, "null argument");
     const ppl_dedisp_job job{p, d_in, d_out};
+    if (!p->ownTile) return run_default(&job, 1, stream_of(stream));
     return run_jobs(&job, 1, Shape{p->nd, p->nt, p->cb, p->rw}, stream_of(stream));
 }
 
@@ -1816,6 +1977,7 @@ extern "C" int ppl_dedisperse_batch(const ppl_dedisp_job* jobs, int n, int tileD
         if (rc != PPL_OK) return rc;
         return run_jobs(jobs, n, s, stream_of(stream));
     }
+    if (!jobs[0].plan->ownTile) return run_default(jobs, n, stream_of(stream));
     // job 0's own tile; when that is a ring tile some other job's delay
     // spread does not fit (a refusal before any launch), the same tile with
     // one-sample reads
@@ -1830,51 +1992,19 @@ extern "C" int ppl_dedisp_autotune_batch(const ppl_dedisp_job* jobs, int n, int 
 {
     PPL_CHECK_ARG(jobs && n >= 1 && tileDM && tileT && chanBlock && readBytes, "null argument");
     PPL_CHECK_ARG(jobs[0].plan, "job 0: null plan");
-    if (reps < 1) reps = 1;
-    hipStream_t st = stream_of(stream);
-    hipEvent_t e0, e1;
-    PPL_HIP(hipEventCreate(&e0));
-    PPL_HIP(hipEventCreate(&e1));
-    const int cbs[] = {1, 2, 4, 8, 16};
-    float best = 1e30f;
-    Shape bestShape{0, 0, 0};
-    for (const Shape& base : kShapes) {
-        if (!shape_for(base, jobs[0].plan->cfg.dtype)) continue;
-        for (int cb : cbs) {
-            const Shape s{base.nd, base.nt, cb, base.rw};
-            bool fits = true;
-            for (int k = 0; k < n && fits; ++k) {
-                DDJob J{};
-                size_t lds = 0;
-                fits = jobs[k].plan && make_job(jobs[k].plan, s, jobs[k].d_in, jobs[k].d_out, J, &lds) == PPL_OK &&
-                       J.CB >= cb;
-            }
-            if (!fits || run_jobs(jobs, n, s, st) != PPL_OK) continue;  // warm
-            PPL_HIP(hipEventRecord(e0, st));
-            for (int r = 0; r < reps; ++r)
-                if (run_jobs(jobs, n, s, st) != PPL_OK) break;
-            PPL_HIP(hipEventRecord(e1, st));
-            PPL_HIP(hipEventSynchronize(e1));
-            float ms = 0.0f;
-            PPL_HIP(hipEventElapsedTime(&ms, e0, e1));
-            ms /= reps;
-            if (ms < best) {
-                best = ms;
-                bestShape = s;
-            }
-        }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    if (bestShape.nd == 0) {
+    Shape best;
+    float ms = 0.0f;
+    const int rc = fastest_shape(jobs, n, !jobs[0].plan->ownTile, reps, stream_of(stream), &best, &ms);
+    if (rc != PPL_OK) return rc;
+    if (std::isinf(ms)) {
         set_error("autotune: no tile shape fits every job");
         return PPL_E_CONFIG;
     }
-    *tileDM = 4 * bestShape.nd;
-    *tileT = 64 * bestShape.nt;
-    *chanBlock = bestShape.cb;
-    *readBytes = bestShape.rw;
-    if (best_ms) *best_ms = best;
+    *tileDM = 4 * best.nd;
+    *tileT = 64 * best.nt;
+    *chanBlock = best.cb;
+    *readBytes = best.rw;
+    if (best_ms) *best_ms = ms;
     return PPL_OK;
 }
 

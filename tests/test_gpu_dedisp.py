@@ -61,6 +61,46 @@ def test_f32_bit_exact_ragged(orc, ppl, shape, reads):
     assert np.array_equal(out, orc.dedisperse(x, d, p["nout"]))
 
 
+# (channels, trials, delay per trial in the last channel, output samples): the
+# register-window kernel's shapes and stagings, with remainders of trials,
+# samples, channels and rounds of channels at each
+WINDOW_SHAPES = [
+    # long tiles (1280 samples; 1536 in FP16): one, two and four pieces a lane,
+    # shared windows, windows of a trial's own, and both in one plan
+    (7, 2113, 1.7, 5200), (18, 2113, 6.3, 5200), (3, 2113, 31.0, 5200), (2, 2113, 101.0, 5200),
+    # 768 samples: a row a wave, and split rows
+    (9, 1093, 5.9, 5100), (5, 1093, 23.0, 5100), (1, 1093, 90.0, 5100),
+    # 256 samples (512 in FP16): rows of two and four pieces, and split ones
+    (26, 37, 3.0, 700), (17, 37, 14.0, 700), (8, 37, 50.0, 700), (11, 33, 200.0, 700), (1, 1, 0.0, 224)]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+@pytest.mark.parametrize("n_chan,tdms,slope,n_out", WINDOW_SHAPES)
+def test_window_kernel_bit_exact(orc, ppl, dtype, n_chan, tdms, slope, n_out):
+    """Plans without a tile of their own, whose rows are whole 16-byte pieces:
+    every sum equals the oracle's channel-order sum, infinities and NaN at
+    the end of a row included; the same input 4 bytes off a 16-byte boundary
+    (the one-word and ring kernels) gives the same."""
+    tsamp, fch1, foff = 0.00032768, 150.0, -0.05
+    f = fch1 + foff * (n_chan - 1)
+    shift = 4148.741601 * (1.0 / f / f - 1.0 / fch1 / fch1) if n_chan > 1 else 1.0
+    nsamp = (int(slope * (tdms - 1)) + n_out + 240) // 16 * 16
+    cfg = dict(n_chan=n_chan, nsamp_buf=nsamp, tdms=tdms, dm_low=0.0, dm_step=slope * tsamp / shift, tsamp=tsamp,
+               fch1=fch1, foff=foff)
+    rng = np.random.default_rng(n_chan + tdms)
+    x = rng.normal(size=(n_chan, nsamp)).astype(np.float32)
+    x[-1, -1], x[0, -1] = np.inf, np.nan
+    p, d = _oracle(orc, x, cfg)
+    host = x if dtype == "f32" else orc.f32_to_f16_bits(x)
+    exp = orc.dedisperse(host, d, p["nout"])
+    dev = torch.from_numpy(x if dtype == "f32" else host.view(np.float16)).cuda()
+    plan = ppl.DedispPlan(**cfg, dtype=dtype)
+    assert np.array_equal(plan.run(dev).cpu().numpy(), exp, equal_nan=True)
+    off = torch.empty(dev.numel() + 8, dtype=dev.dtype, device="cuda")[4 // dev.element_size():][:dev.numel()]
+    off.copy_(dev.view(-1))
+    assert np.array_equal(plan.run(off).cpu().numpy(), exp, equal_nan=True)
+
+
 def test_known_answer_dm10(ppl):
     """DedispersionModuleTest.cpp:167-168: dmAmplitude(0, 10) == nSub*nCh."""
     nsub, nch = 32, 64
