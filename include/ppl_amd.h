@@ -104,18 +104,19 @@ typedef struct {
  * builds the FP32 delay table on the host from the FP64 shift table exactly
  * as the reference (:152-162, DedispersionKernel.cu:29,36), uploads it and
  * picks the kernel: for FP32 and FP16 rows of whole 16-byte pieces the
- * register-window kernel, in a shape that its sizes call for, and beside it a
- * tile for the others (input that is not 16-byte aligned, a tile set later):
- * for FP32 the ring kernel at 32 trials x 512 samples where a tile's delay
- * spread fits its staged row, else (and for f16 and u8) the one-word kernel at
- * 32 (or fewer) trials x 512.  ppl_dedisp_info reports that tile.  Fails with PPL_E_CONFIG when nsampBuf <= maxshift
+ * register-window kernel, in a shape that its sizes call for, for u8 the group
+ * kernel where neighbouring channels' delays keep together over 48 trials, and
+ * beside it a tile for the others (input that is not 16-byte aligned, a tile
+ * set later): the ring kernel at 32 trials x 512 samples (FP32, and u8 without
+ * the group kernel) where a tile's delay spread fits its staged row, else the
+ * one-word kernel at 32 (or fewer) trials x 512.  ppl_dedisp_info reports that tile.  Fails with PPL_E_CONFIG when nsampBuf <= maxshift
  * (the module's throw at :175-178), when dmStep < 0 (delays would decrease
  * with the trial index) or when a delayed read would leave the channel row. */
 int ppl_dedisp_plan_create(ppl_dedisp_plan** plan, const ppl_dedisp_config* cfg);
 int ppl_dedisp_plan_destroy(ppl_dedisp_plan* plan);
 int ppl_dedisp_plan_info(const ppl_dedisp_plan* plan, ppl_dedisp_info* info);
 /* Override the DM x time tile (the autotuner's hook); 0 keeps the default.  A
- * plan whose tile was set runs that tile and not the window kernel. */
+ * plan whose tile was set runs that tile and not the window or group kernel. */
 int ppl_dedisp_set_tile(ppl_dedisp_plan* plan, int tileDM, int tileT);
 /* Same with the number of channels staged per LDS block (0: as many as fit). */
 int ppl_dedisp_set_shape(ppl_dedisp_plan* plan, int tileDM, int tileT, int chanBlock);

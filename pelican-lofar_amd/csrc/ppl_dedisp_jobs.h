@@ -51,6 +51,9 @@ __device__ __forceinline__ void wait_vmcnt()
 
 __device__ __forceinline__ void bare_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
+// A barrier after this wave's LDS writes have landed.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // LDS address (byte offset in the workgroup's LDS) of a __shared__ pointer.
 __device__ __forceinline__ uint32_t lds_addr(const void* p)
 {

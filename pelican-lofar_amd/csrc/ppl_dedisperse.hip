@@ -16,6 +16,7 @@
 // and quarter the bytes per add.
 #include "ppl_internal.h"
 #include "ppl_dedisp_jobs.h"
+#include "ppl_dedisp_u8group.h"
 #include "ppl_dedisp_window.h"
 
 #include <algorithm>
@@ -45,6 +46,7 @@ struct ppl_dedisp_plan {
     // take that kernel), shape (an index of kWinShapes) and staging
     int4* d_win = nullptr;
     int winShape = 0, winStaging = 0;
+    int32_t* d_u8g = nullptr;  // the u8 group kernel's table (ppl_dedisp_u8group.h), or null
     bool ownTile = false;  // a tile was set (by the caller or the autotuner)
     int defNd = 8, defNt = 8, defRw = 4;  // the tile the plan started with
     // u8 series, built on first use: per trial dm, the number of channels
@@ -52,6 +54,7 @@ struct ppl_dedisp_plan {
     // lenOff[tdms] is the table's length
     int32_t* d_lenOff = nullptr;
     uint16_t* d_lenTab = nullptr;
+    int lenMax = 0;  // entries of the longest trial
 };
 
 namespace {
@@ -914,9 +917,6 @@ __device__ __forceinline__ void dma_dword_s(const void* g, uint32_t laneBytes, u
                  : "memory");
 }
 
-// A barrier after this wave's LDS writes have landed.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // Eight dword reads, two from each of four addresses (the second 256 bytes
 // on: the q = 1 dword), waiting for them before the block ends.
 __device__ __forceinline__ void lds_read4x2(const uint32_t (&a)[4], uint32_t (&v)[8])
@@ -1518,17 +1518,20 @@ const WinEntry kWinShapes[] = {win_entry<WinF32>(), win_entry<WinF32Short>(), wi
                                win_entry<WinF16>(), win_entry<WinF16Small>()};
 
 // Jobs whose plan has no tile set run the kernel that its sizes call for: the
-// window kernel where the plan has its table and the input is 16-byte aligned
-// (rows then start on 16 bytes: the table is only built for such row
-// lengths), else the plan's first tile.  One launch per kernel and tile.
-bool takes_window(const ppl_dedisp_job& jb)
+// window kernel (FP32, FP16) or the group kernel (u8) where the plan has its
+// table and the input is 16-byte aligned (the tables are only built for sizes
+// that then keep to whole 16 bytes), else the plan's first tile.  One launch
+// per kernel and tile.
+bool takes_table(const ppl_dedisp_job& jb)
 {
-    return (reinterpret_cast<uintptr_t>(jb.d_in) & 15) == 0 && jb.plan->d_win;
+    return (reinterpret_cast<uintptr_t>(jb.d_in) & 15) == 0 && (jb.plan->d_win || jb.plan->d_u8g);
 }
 
-int run_window(const ppl_dedisp_job* const* jobs, int n, hipStream_t st)
+int run_tables(const ppl_dedisp_job* const* jobs, int n, hipStream_t st)
 {
+    const bool u8 = jobs[0]->plan->d_u8g != nullptr;
     const WinEntry& W = kWinShapes[jobs[0]->plan->winShape];
+    const int TD = u8 ? kU8gTD : kWinTD, TT = u8 ? kU8gTT : W.TT;
     DDBatch B{};
     B.n = n;
     long blocks = 0;
@@ -1537,19 +1540,24 @@ int run_window(const ppl_dedisp_job* const* jobs, int n, hipStream_t st)
         DDJob& J = B.job[k];
         J.in = jobs[k]->d_in;
         J.out = jobs[k]->d_out;
-        J.delayT = reinterpret_cast<const int32_t*>(p->d_win);
+        J.delayT = u8 ? p->d_u8g : reinterpret_cast<const int32_t*>(p->d_win);
         J.nChan = (int)p->cfg.nChan;
         J.nsamp = (int)p->cfg.nsampBuf;
         J.tdms = (int)p->cfg.tdms;
         J.nOut = p->nOut;
-        J.nDMTiles = (J.tdms + kWinTD - 1) / kWinTD;
-        const long tiles = (long)J.nDMTiles * ((J.nOut + W.TT - 1) / W.TT);
+        J.CB = u8g_capacity(J.nChan);
+        J.nDMTiles = (J.tdms + TD - 1) / TD;
+        const long tiles = (long)J.nDMTiles * ((J.nOut + TT - 1) / TT);
         PPL_CHECK_ARG(blocks + tiles + kXcds < (1L << 31), "grid too large");
         J.nTiles = (int)tiles;
         J.blockStart = (int)blocks;
         blocks += (tiles + kXcds - 1) / kXcds * kXcds;
     }
-    hipLaunchKernelGGL(W.kernel[jobs[0]->plan->winStaging], dim3((unsigned)blocks), dim3(64 * kWinWaves), 0, st, B);
+    const dim3 grid((unsigned)blocks);
+    if (u8)
+        hipLaunchKernelGGL(dedisperse_u8_group_kernel, grid, dim3(64 * (kU8gSum + kU8gBuild)), 0, st, B);
+    else
+        hipLaunchKernelGGL(W.kernel[jobs[0]->plan->winStaging], grid, dim3(64 * kWinWaves), 0, st, B);
     PPL_LAUNCHED();
     return PPL_OK;
 }
@@ -1570,16 +1578,16 @@ int run_default(const ppl_dedisp_job* jobs, int n, hipStream_t st)
     bool done[kMaxDDJobs] = {};
     for (int k = 0; k < n; ++k) {
         const ppl_dedisp_plan* p = jobs[order[k]].plan;
-        if (done[order[k]] || !takes_window(jobs[order[k]])) continue;
+        if (done[order[k]] || !takes_table(jobs[order[k]])) continue;
         const ppl_dedisp_job* same[kMaxDDJobs];
         int m = 0;
         for (int i = k; i < n; ++i) {
             const ppl_dedisp_job& jb = jobs[order[i]];
-            if (!takes_window(jb) || jb.plan->winShape != p->winShape || jb.plan->winStaging != p->winStaging) continue;
+            if (!takes_table(jb) || jb.plan->winShape != p->winShape || jb.plan->winStaging != p->winStaging) continue;
             done[order[i]] = true;
             same[m++] = &jb;
         }
-        const int rc = run_window(same, m, st);
+        const int rc = run_tables(same, m, st);
         if (rc != PPL_OK) return rc;
     }
     for (int k = 0; k < n; ++k) {
@@ -1694,6 +1702,47 @@ int window_table(ppl_dedisp_plan* p)
     return PPL_OK;
 }
 
+// The u8 group kernel's table, where its tiles' delay spread fits a row, the
+// input ends on 16 bytes, no tile needs more passes than its capacity and,
+// where the ring kernel fits, the mean is below two passes a group (where the
+// two take the same time).  Without it a plan takes the ring kernel if its
+// 32-trial tiles fit that (the conditions of make_job), else the one-word tile,
+// and so do plans of fewer tiles than half the CUs, where the one-word kernel's
+// smaller tiles are as fast.
+int u8_kernel(ppl_dedisp_plan* p)
+{
+    if (p->cfg.dtype != PPL_U8) return PPL_OK;
+    const int tdms = (int)p->cfg.tdms, nChan = (int)p->cfg.nChan, nsamp = (int)p->cfg.nsampBuf;
+    const long total = (long)nChan * nsamp;
+    const long dmTiles = (tdms + kU8gTD - 1) / kU8gTD;
+    if (dmTiles * ((p->nOut + kU8gTT - 1) / kU8gTT) < 128) return PPL_OK;
+    const bool ring = total < (1L << 31) && total % 4 == 0 && (span_of(p, 32) + 3) / 4 + 512 / 4 <= kU8CopyDw - 1;
+    if (total % 16 == 0 && total < (1L << 31) && tile_span(p->delays, tdms, nChan, kU8gTD) <= kU8gSpan) {
+        const int nTiles = (tdms + kU8gTD - 1) / kU8gTD, nGroups = (nChan + 3) / 4, capacity = u8g_capacity(nChan);
+        PPL_CHECK_ARG((long)nTiles * nGroups < (1L << 31), "u8 group table too large");
+        PPL_HIP(hipMalloc(&p->d_u8g, u8g_table_bytes(nTiles, nChan)));
+        PPL_HIP(hipMemset(p->d_u8g, 0, (size_t)nTiles * sizeof(int32_t)));
+        hipLaunchKernelGGL(u8g_table_kernel, dim3((unsigned)((nTiles * nGroups + 3) / 4)), dim3(256), 0, nullptr,
+                           p->d_delayT, nChan, nsamp, tdms, p->tdmsPad, nTiles, capacity, p->d_u8g);
+        PPL_LAUNCHED();
+        std::vector<int32_t> passes(nTiles);
+        PPL_HIP(hipMemcpy(passes.data(), p->d_u8g, nTiles * sizeof(int32_t), hipMemcpyDeviceToHost));
+        long sum = 0;
+        for (int v : passes) sum += v;
+        if (*std::max_element(passes.begin(), passes.end()) <= capacity && (!ring || sum < 2L * nTiles * nGroups))
+            return PPL_OK;
+        PPL_HIP(hipFree(p->d_u8g));
+        p->d_u8g = nullptr;
+    }
+    if (ring) {
+        p->nd = p->nt = p->defNd = p->defNt = 8;
+        p->rw = p->defRw = 16;
+        const int32_t* tab = nullptr;
+        return ring_table(p, 32, &tab);  // now, not in a first launch that may be captured
+    }
+    return PPL_OK;
+}
+
 }  // namespace
 
 extern "C" int ppl_dedisp_plan_create(ppl_dedisp_plan** plan, const ppl_dedisp_config* cfg)
@@ -1790,6 +1839,7 @@ extern "C" int ppl_dedisp_plan_create(ppl_dedisp_plan** plan, const ppl_dedisp_c
     p->defRw = p->rw;
     int rc = upload_delays(p);
     if (rc == PPL_OK) rc = window_table(p);
+    if (rc == PPL_OK) rc = u8_kernel(p);
     if (rc != PPL_OK) {
         ppl_dedisp_plan_destroy(p);
         return rc;
@@ -1805,6 +1855,7 @@ extern "C" int ppl_dedisp_plan_destroy(ppl_dedisp_plan* plan)
     for (int32_t* t : plan->d_ring)
         if (t) (void)hipFree(t);
     if (plan->d_win) (void)hipFree(plan->d_win);
+    if (plan->d_u8g) (void)hipFree(plan->d_u8g);
     if (plan->d_lenOff) (void)hipFree(plan->d_lenOff);
     if (plan->d_lenTab) (void)hipFree(plan->d_lenTab);
     delete plan;
@@ -2144,10 +2195,105 @@ __global__ __launch_bounds__(1024) void exceptional_rows_kernel(const float* __r
         if (rowOff[i] != 0.0f) rows[o++] = i;
 }
 
+// The same sums as u8_series_kernel below where a trial's counts fit LDS as
+// floats.  A workgroup of eight waves holds them for 8192 samples of one trial,
+// reversed and with 1024 zeros on both sides, so that for a row the counts of a
+// wave's 1024 samples (16 a lane, 64 apart) are reads at fixed distances
+// with no test of the range; a count of zero adds nothing, which a product
+// with a finite offset does by itself.  The exceptional rows that reach the
+// samples are gathered in LDS, 2048 rows at a time in increasing order, so no
+// list of them is kept in memory.
+constexpr int kSeriesJ = 16, kSeriesPad = 64 * kSeriesJ, kSeriesTT = 8 * kSeriesPad, kSeriesRows = 2048;
+constexpr int kSeriesMaxLen = 33792;  // counts of a trial: 156 KB of LDS with the zeros and the rows
+inline size_t series_lds_bytes(int lenMax) { return sizeof(float) * (lenMax + 2 * kSeriesPad + 2 * kSeriesRows + 32); }
+__global__ __launch_bounds__(512) void u8_series_lds_kernel(const int32_t* __restrict__ sums,
+                                                            const float* __restrict__ rowOff, int nsamp,
+                                                            const uint16_t* __restrict__ lenTab,
+                                                            const int32_t* __restrict__ lenOff, int nOut, int offset,
+                                                            float scale, float* __restrict__ out)
+{
+    extern __shared__ float series_lds[];
+    int* rowAt = reinterpret_cast<int*>(series_lds);       // [kSeriesRows]
+    float* rowVal = series_lds + kSeriesRows;              // [kSeriesRows]
+    int* hits = reinterpret_cast<int*>(rowVal + kSeriesRows);  // [4 reads][8 waves]
+    float* counts = rowVal + kSeriesRows + 32;             // counts[kSeriesPad + dmax - k] of delay k
+    const int dm = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int T0 = blockIdx.x * kSeriesTT, t0 = T0 + kSeriesPad * wave;
+    const int base = lenOff[dm];
+    const int dmax = lenOff[dm + 1] - base - 1;
+    for (int i = tid; i < dmax + 1 + 2 * kSeriesPad; i += 512) {
+        const int k = dmax + kSeriesPad - i;
+        counts[i] = k >= 0 && k <= dmax ? (float)lenTab[base + k] : 0.0f;
+    }
+    float corr[kSeriesJ];
+#pragma unroll
+    for (int j = 0; j < kSeriesJ; ++j) corr[j] = 0.0f;
+    const int end = min(nsamp, min(T0 + kSeriesTT, nOut) + dmax);  // past the last row that reaches the samples
+    for (int e0 = T0; e0 < end; e0 += kSeriesRows) {
+        float off[4];
+        uint64_t hit[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = e0 + 512 * i + tid;
+            off[i] = e < end ? rowOff[e] : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            hit[i] = __ballot(off[i] != 0.0f);
+            if (lane == 0) hits[8 * i + wave] = __builtin_popcountll(hit[i]);
+        }
+        __syncthreads();  // the hits; the first time round the counts too
+        int incl = lane < 32 ? hits[lane] : 0;
+        for (int d = 1; d < 32; d <<= 1) {
+            const int y = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += y;
+        }
+        const int n = __shfl(incl, 31, 64);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int before = 8 * i + wave == 0 ? 0 : __shfl(incl, max(8 * i + wave - 1, 0), 64);
+            if (off[i] != 0.0f) {
+                const int at = before + __builtin_popcountll(hit[i] & ((1ull << lane) - 1));
+                rowAt[at] = e0 + 512 * i + tid;
+                rowVal[at] = off[i];
+            }
+        }
+        __syncthreads();  // the rows
+        for (int i = 0; i < n; ++i) {
+            const int e = __builtin_amdgcn_readfirstlane(rowAt[i]);
+            if (e < t0) continue;
+            if (e > t0 + kSeriesPad - 1 + dmax) break;
+            const float v = rowVal[i];
+            // sample t0 + lane + 64 j has delay e - t; e - t0 is in 0 .. dmax + 1023
+            const float* c = counts + (kSeriesPad + dmax - (e - t0)) + lane;
+            if (__builtin_isfinite(v)) {
+#pragma unroll
+                for (int j = 0; j < kSeriesJ; ++j) corr[j] = corr[j] + v * c[64 * j];
+            } else {
+#pragma unroll
+                for (int j = 0; j < kSeriesJ; ++j)
+                    if (c[64 * j] != 0.0f) corr[j] = corr[j] + v * c[64 * j];
+            }
+        }
+        __syncthreads();  // the rows are done with
+    }
+#pragma unroll
+    for (int j = 0; j < kSeriesJ; ++j) {
+        const int t = t0 + lane + 64 * j;
+        if (t < nOut) {
+            const size_t i = (size_t)dm * nOut + t;
+            out[i] = (float)(sums[i] - offset) * scale + corr[j];
+        }
+    }
+}
+
 // out[dm][t] = float(S - offset) * scale, plus, for every exceptional row e
 // with 0 <= e - t <= maxdelay(dm) in increasing order, rowOff[e] times the
 // number of channels whose delay is e - t (each product rounded, then
-// added).  One workgroup per (256 samples, trial).
+// added).  One workgroup per (256 samples, trial): trials with more counts than
+// u8_series_lds_kernel holds.
 __global__ __launch_bounds__(256) void u8_series_kernel(const int32_t* __restrict__ sums,
                                                         const float* __restrict__ rowOff,
                                                         const int* __restrict__ rows, const int* __restrict__ nRowsP,
@@ -2196,6 +2342,7 @@ int len_table(const ppl_dedisp_plan* cp, const int32_t** lenOff, const uint16_t*
             off[dm] = (int32_t)total;
             int dmax = 0;
             for (int c = 0; c < nChan; ++c) dmax = std::max(dmax, p->delays[(size_t)dm * nChan + c]);
+            p->lenMax = std::max(p->lenMax, dmax + 1);
             total += dmax + 1;
             PPL_CHECK_ARG(total < (1L << 31), "u8 series: channel-count table too large");
         }
@@ -2240,6 +2387,16 @@ extern "C" int ppl_dedisp_u8_series(const ppl_dedisp_plan* p, const int32_t* d_s
     if (rc != PPL_OK) return rc;
     hipStream_t st = stream_of(stream);
     const int nsamp = (int)p->cfg.nsampBuf;
+    // One launch, no scratch, from 2^22 series samples on (LOFAR-size beam with
+    // 0.5 % of rows exceptional: 2.95 -> 1.2 ms); small series and trials whose
+    // counts do not fit LDS list the rows first.
+    if (p->lenMax <= kSeriesMaxLen && (long)p->cfg.tdms * p->nOut >= (1L << 22)) {
+        dim3 grid(cdiv((unsigned)p->nOut, kSeriesTT), p->cfg.tdms);
+        hipLaunchKernelGGL(u8_series_lds_kernel, grid, dim3(512), series_lds_bytes(p->lenMax), st, d_sums,
+                           d_rowOffsets, nsamp, lenTab, lenOff, p->nOut, (int)(128 * p->cfg.nChan), scale, d_out);
+        PPL_LAUNCHED();
+        return PPL_OK;
+    }
     int* rows = nullptr;
     PPL_HIP(hipMallocAsync((void**)&rows, sizeof(int) * ((size_t)nsamp + 1), st));
     hipLaunchKernelGGL(exceptional_rows_kernel, dim3(1), dim3(1024), 0, st, d_rowOffsets, nsamp, rows + 1, rows);

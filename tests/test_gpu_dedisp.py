@@ -101,6 +101,70 @@ def test_window_kernel_bit_exact(orc, ppl, dtype, n_chan, tdms, slope, n_out):
     assert np.array_equal(plan.run(off).cpu().numpy(), exp, equal_nan=True)
 
 
+# (channels, trials, samples of delay per trial in the last channel, output
+# samples) for the u8 group kernel, which takes 128 tiles of 48 trials x 1024
+# samples and more: ends of groups of four channels, of tiles and of the 64
+# passes between widenings; more passes than groups where the delays are steep;
+# the last with too many, which the ring kernel takes
+U8_GROUP_SHAPES = [(1, 3100, 0.0, 1030), (2, 5, 0.5, 130900), (3, 48, 1.0, 131200), (5, 49, 4.0, 65600),
+                   (53, 97, 6.3, 43100), (64, 150, 0.02, 33000), (258, 50, 2.0, 65600), (131, 96, 10.0, 65600),
+                   (6, 97, 9.9, 43100)]
+
+
+@pytest.mark.parametrize("n_chan,tdms,slope,n_out", U8_GROUP_SHAPES)
+@pytest.mark.parametrize("full", [False, True])
+def test_u8_group_kernel_exact(orc, ppl, n_chan, tdms, slope, n_out, full):
+    """u8 plans without a tile of their own: the oracle's sums, with every
+    value at 255 too (the 16-bit partial sums at their largest), and the same
+    from an input 4 bytes off a 16-byte boundary (the ring and one-word
+    kernels)."""
+    tsamp, fch1 = 0.00032768, 150.0
+    foff = -0.05 if n_chan < 100 else -20.0 / n_chan
+    f = fch1 + foff * (n_chan - 1)
+    shift = 4148.741601 * (1.0 / f / f - 1.0 / fch1 / fch1) if n_chan > 1 else 1.0
+    nsamp = (int(slope * (tdms - 1)) + n_out + 240) // 16 * 16
+    cfg = dict(n_chan=n_chan, nsamp_buf=nsamp, tdms=tdms, dm_low=0.0, dm_step=slope * tsamp / shift, tsamp=tsamp,
+               fch1=fch1, foff=foff)
+    p, d = _oracle(orc, None, cfg)
+    if full:
+        x = np.full((n_chan, nsamp), 255, np.uint8)
+    else:
+        x = np.random.default_rng(n_chan).integers(0, 256, size=(n_chan, nsamp), dtype=np.uint8)
+    exp = orc.dedisperse(x, d, p["nout"])
+    dev = torch.from_numpy(x).cuda()
+    plan = ppl.DedispPlan(**cfg, dtype="u8")
+    assert np.array_equal(plan.run(dev).cpu().numpy(), exp)
+    off = torch.empty(dev.numel() + 8, dtype=torch.uint8, device="cuda")[4:4 + dev.numel()]
+    off.copy_(dev.view(-1))
+    assert np.array_equal(plan.run(off).cpu().numpy(), exp)
+
+
+@pytest.mark.parametrize("maxdelay", [40, 5000, 15600, 32800, 36500])
+def test_u8_series_delays_of_any_length(orc, ppl, maxdelay):
+    """u8 series (from 2^22 samples on) where a trial's channel counts fit LDS
+    (up to 33792 of them) and where they do not; offsets at the first and last rows, side by side,
+    and infinite."""
+    n_chan, tdms, tsamp, fch1, foff = 48, 130, 0.00032768, 150.0, -0.05
+    f = fch1 + foff * (n_chan - 1)
+    shift = 4148.741601 * (1.0 / f / f - 1.0 / fch1 / fch1)
+    nsamp = (maxdelay + 34000) // 16 * 16
+    cfg = dict(n_chan=n_chan, nsamp_buf=nsamp, tdms=tdms, dm_low=maxdelay * tsamp / shift,
+               dm_step=7.3 * tsamp / shift, tsamp=tsamp, fch1=fch1, foff=foff)
+    p, d = _oracle(orc, None, cfg)
+    rng = np.random.default_rng(maxdelay)
+    q = rng.integers(0, 256, size=(n_chan, nsamp), dtype=np.uint8)
+    off = np.zeros(nsamp, np.float32)
+    at = rng.choice(nsamp, size=60, replace=False)
+    off[at] = -2500.0 - 100.0 * rng.random(60)
+    off[[0, 1, 2, nsamp - 1, nsamp - 2]] = [-3.5, 7.25, -1e30, 2.0, -0.125]
+    off[nsamp // 2] = -np.inf
+    plan = ppl.DedispPlan(**cfg, dtype="u8")
+    assert tdms * plan.nout >= 1 << 22
+    sums = plan.run(torch.from_numpy(q).cuda())
+    got = plan.u8_series(sums, torch.from_numpy(off).cuda(), 0.25).cpu().numpy()
+    assert np.array_equal(got, orc.u8_series(sums.cpu().numpy(), off, d, p["nout"], np.float32(0.25)))
+
+
 def test_known_answer_dm10(ppl):
     """DedispersionModuleTest.cpp:167-168: dmAmplitude(0, 10) == nSub*nCh."""
     nsub, nch = 32, 64
