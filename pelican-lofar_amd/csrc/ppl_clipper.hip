@@ -28,6 +28,7 @@
 #include <cmath>
 #include <map>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -224,6 +225,7 @@ __device__ __forceinline__ float ring_front(RingView r, int start) { return r.bu
 
 constexpr int kWalkThreads = 512;
 constexpr int kStage = 512;      // spectra whose precomputed records are staged in LDS at a time
+constexpr int kStagePad = 16;     // a fold over the staged spectra reads and writes up to that far past them
 constexpr int kRowChunk = 8192;  // bins of one spectrum staged in LDS for the ordered sums
 constexpr int kMaxBinsWalk = 32768;  // bins per spectrum the walk supports (kept-bin mask in LDS)
 static_assert(kStage == kWalkThreads, "stage scans use one thread per staged spectrum");
@@ -267,7 +269,24 @@ enum {
     PRE_REJ = 4,      // (walk) the mask in force rejects the spectrum for certain: 4 bad bands or more
     PRE_ONE = 8,       // exactly one channel undecided: its decision picks one of two records
     PRE_PREDKEPT = 16, // (PRE_ONE) the undecided channel is kept at the predicting state
-    PRE_TOLREJ = 32    // (walk) the mask keeps it, but its mean exceeds the tolerance at the stage-start state
+    PRE_TOLREJ = 32,   // (walk) the mask keeps it, but its mean exceeds the tolerance at the stage-start state
+    PRE_MANY = 64      // 2 to kUndMax channels undecided, and rejected whichever way they go: an UndRec is there
+};
+// The undecided channels of a spectrum with a few of them that has 4 bad
+// bands or more even with all of them kept (broadband interference clips most
+// of a spectrum and leaves a few channels near the threshold).  Its decision
+// is certain; only its share of bad channels waits for them, which the walk
+// counts at the spectrum's own state without reading the spectrum again.
+// In 52640 spectra of a LOFAR beam 242 are such, with 2 to 16 open channels
+// each: a pass of the workgroup over the whole spectrum took 8.3 us and ended
+// a speculative block, 173 spectra long on average; with them in the blocks
+// (511 long) the walk takes 2.85 ms instead of 6.0.
+constexpr int kUndMax = 16;
+struct UndRec {
+    int n;        // undecided channels
+    int nKept;    // channels kept over the whole box
+    int bin[kUndMax];
+    float val[kUndMax];
 };
 
 constexpr int kMaxVer = 64;  // last-good versions kept per run for the apply pass
@@ -507,6 +526,7 @@ struct BeamState {
     const unsigned* kill;  // killed bins of the run map (bit mask), or null
     Box* box;
     PreRec* pre;
+    UndRec* und;  // beside pre: written for PRE_MANY spectra only
     LearnRec* learn;
     SpecRec* rec;
     float2* stats;
@@ -609,14 +629,15 @@ __device__ __forceinline__ void pre_rows(const BatchIO& io)
     const float* __restrict__ bpHi = bs.bpHi;
     const float* __restrict__ lastGood = bs.lastGood;
     PreRec* __restrict__ pre = bs.pre;
+    UndRec* __restrict__ undRec = bs.und;
     const int nT = io.nT[beam], subLen = io.subLen[beam], ldMode = io.ldMode[beam];
     __shared__ float vals[2][kPreRows][kTileBins + 1];
     // the same rows with the undecided channels kept, for rows with one
     __shared__ float valsK[2][kPreRows][kTileBins + 1];
     __shared__ int cnt[kPreRows][8];
     __shared__ int rowFlags[kPreRows];
-    __shared__ int undCnt[kPreRows], undBinS[kPreRows];
-    __shared__ float undValS[kPreRows];
+    __shared__ int undCnt[kPreRows], undBand[kPreRows][8], undBinS[kPreRows][kUndMax];
+    __shared__ float undValS[kPreRows][kUndMax];
     const int tStart = S->tNext;
     if (tStart >= nT) return;
     const Box bx = *box;
@@ -631,7 +652,10 @@ __device__ __forceinline__ void pre_rows(const BatchIO& io)
     const float invCpb = 1.0f / (float)cpb;
     const long rowStride = (long)nBins * nPol;
     const int nTiles = (nBins + kTileBins - 1) / kTileBins;
-    for (int i = tid; i < kPreRows * 8; i += kTileThreads) (&cnt[0][0])[i] = 0;
+    for (int i = tid; i < kPreRows * 8; i += kTileThreads) {
+        (&cnt[0][0])[i] = 0;
+        (&undBand[0][0])[i] = 0;
+    }
     if (tid < kPreRows) {
         rowFlags[tid] = 0;
         undCnt[tid] = 0;
@@ -684,10 +708,13 @@ __device__ __forceinline__ void pre_rows(const BatchIO& io)
                     valsK[buf][r][lane * 4 + j] = (keep[j] || uj) ? v : 0.0f;
                 }
                 if (uj) {
-                    // rare: with two or more the bin and value are not used
-                    atomicAdd(&undCnt[r], 1);
-                    undBinS[r] = i + j;
-                    undValS[r] = v;
+                    // rare; those past kUndMax are only counted
+                    const int at = atomicAdd(&undCnt[r], 1);
+                    atomicAdd(&undBand[r][band[j]], 1);
+                    if (at < kUndMax) {
+                        undBinS[r][at] = i + j;
+                        undValS[r][at] = v;
+                    }
                 }
             }
             for (int b = bandLo; b <= bandHi; ++b) {
@@ -734,19 +761,41 @@ __device__ __forceinline__ void pre_rows(const BatchIO& io)
         pre[k0 + lane].mean = r.mean;
         pre[k0 + lane].fracInc = r.fracInc;
         pre[k0 + lane].badBands = r.badBands;
-        if (!(r.flags & PRE_UND) || undCnt[lane] != 1) pre[k0 + lane].flags = r.flags;
+        const int nu = undCnt[lane];
+        if (nu != 1) {
+            if (nu > 1 && nu <= kUndMax) {
+                // with every undecided channel kept: more kept channels never
+                // make more bad bands, so 4 or more here hold for any decision
+#pragma unroll
+                for (int b = 0; b < 8; ++b) c[b] += undBand[lane][b];
+                int totalAll, badAll;
+                band_stats(c, nBins, cpb, totalAll, badAll, fracInc);
+                if (badAll >= 4) {
+                    r.flags |= PRE_MANY;
+                    pre[k0 + lane].badBands = badAll;
+                    UndRec& u = undRec[k0 + lane];
+                    u.n = nu;
+                    u.nKept = total;
+                    for (int j = 0; j < nu; ++j) {
+                        u.bin[j] = undBinS[lane][j];
+                        u.val[j] = undValS[lane][j];
+                    }
+                }
+            }
+            pre[k0 + lane].flags = r.flags;
+        }
     } else if (folder && undCnt[foldRow] == 1) {
         // the record with the one undecided channel kept, and the decision
         // it gets at the sub-chunk-start state (steady state: dataModel 0,
         // margin crFactor * rmsRunAve, RFI_Clipper.cpp:305-311)
-        const int row = foldRow, u = undBinS[row];
+        const int row = foldRow, u = undBinS[row][0];
         int c[8];
 #pragma unroll
         for (int b = 0; b < 8; ++b) c[b] = cnt[row][b] + (band_of(u, invCpb) == b ? 1 : 0);
         int total, badBands;
         float fracInc;
         band_stats(c, nBins, cpb, total, badBands, fracInc);
-        const float v = undValS[row];
+        const float v = undValS[row][0];
         const float bpu = bp_value(bs.terms, K.nTerms, nBins, u, S->params0, K.scale, bs.kill);
         const bool predKept = !((v - 0.0f) - bpu > K.crFactor * S->rmsRunAve);
         PreRec& r = pre[k0 + row];
@@ -858,7 +907,8 @@ __device__ __forceinline__ void learn_rows(const BatchIO& io)
 struct Staged {
     float mean, fracInc;
     int badBands, flags;
-    float meanC, meanFC, rmsFC, pad;
+    float meanC, meanFC, rmsFC;
+    int slot;  // (PRE_MANY) where its undecided channels are staged
 };
 // Staged for a spectrum with one undecided channel (PRE_ONE): the record
 // with that channel kept, the channel, its value and its bandpass terms.
@@ -881,6 +931,34 @@ __device__ __forceinline__ bool var_kept(const VarRec& v, int nTerms, float p0, 
         bp = scale * tot;
     }
     return !((v.undVal - 0.0f) - bp > margin);
+}
+
+// Staged for PRE_MANY spectra: kUndSlots of them a stage (any further one
+// goes to the workgroup), their undecided channels in kUndMax columns each.
+constexpr int kUndSlots = kWalkThreads / kUndMax;  // a thread per channel
+struct UndStage {
+    int k[kUndSlots], n[kUndSlots], nKept[kUndSlots];  // stage index, undecided and kept channels
+    float val[kWalkThreads];
+    unsigned char killed[kWalkThreads];
+    double terms[kMaxParams][kWalkThreads];
+};
+// A staged undecided channel's decision at a state, as in var_kept.
+__device__ __forceinline__ bool und_kept(const UndStage& u, int c, int nTerms, float p0, float scale, float margin)
+{
+    float bp = 0.0f;
+    if (!u.killed[c]) {
+        float tot = 0.0f;
+        tot = (float)((double)tot + (double)p0 * 1.0);
+        for (int j = 0; j < nTerms; ++j) tot = (float)((double)tot + u.terms[j][c]);
+        bp = scale * tot;
+    }
+    return !((u.val[c] - 0.0f) - bp > margin);
+}
+// The bad-channel fraction of a spectrum with that many channels kept (as in
+// band_stats).
+__device__ __forceinline__ float frac_of(int total, int nBins)
+{
+    return (float)(unsigned)(nBins - total) / (float)(unsigned)nBins;
 }
 
 // A sub-chunk's records ahead of its walk: the precompute in the steady
@@ -916,6 +994,7 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
     const unsigned* __restrict__ kill = bst.kill;
     const Box* __restrict__ box = bst.box;
     const PreRec* __restrict__ pre = bst.pre;
+    const UndRec* __restrict__ undRec = bst.und;
     SpecRec* __restrict__ rec = bst.rec;
     const float* __restrict__ bpLo = bst.bpLo;
     const LearnRec* __restrict__ learn = bst.learn;
@@ -936,19 +1015,22 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
     __shared__ Staged stg[kStage];
     // the fold inputs of the staged spectra again, one array per field, so
     // that the single-lane folds read four spectra per LDS access
-    __shared__ __align__(16) float soaMeanFC[kStage], soaMeanC[kStage], soaRmsFC[kStage], soaFracInc[kStage];
+    __shared__ __align__(16) float soaMeanFC[kStage + kStagePad], soaMeanC[kStage], soaRmsFC[kStage + kStagePad],
+        soaFracInc[kStage + kStagePad];
     // the speculative block's records: the precomputed mean (predicted
     // variant for one undecided channel) and whether its mask rejects it
     __shared__ __align__(16) float soaMean[kStage];
     __shared__ __align__(16) int soaRej[kStage];
     __shared__ int lastKept[kStage];  // last spectrum before k the mask keeps, or -1
     __shared__ VarRec var[kStage];
+    __shared__ UndStage us;
+    __shared__ int sh_nMany, sh_refold, waveN[kWalkThreads / 64], waveMin[2][kWalkThreads / 64], waveMax[kWalkThreads / 64];
     // first spectrum at or after k the fast run must not take: undecided
     // channels (blkU), or undecided channels or a last-good fill (blkUF)
     __shared__ int blkU[kStage], blkUF[kStage];
     __shared__ __align__(16) float rowChunk[kRowChunk];
 
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nBins = K.nBins, nCh = K.nCh, nSub = K.nSub, nPol = K.nPol;
     const int cpb = nBins / 8;
     RingView meanR{meanBuf, meanPrefix, K.cap}, rmsR{rmsBuf, rmsPrefix, K.cap};
@@ -956,6 +1038,7 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
         s = *S;
         sh_frontsValid = 0;
         sh_stop = 0;
+        sh_nMany = 0;
     }
     __syncthreads();
     const int tStart = s.tNext;
@@ -1148,6 +1231,13 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
                     cRej = v.badBandsK >= 4;
                 }
                 ++nResolved;
+            } else if (cur.flags & PRE_MANY) {
+                // rejected whichever way they go: only the fraction is open
+                int total = us.nKept[cur.slot];
+                for (int c = 0; c < us.n[cur.slot]; ++c)
+                    total += und_kept(us, cur.slot * kUndMax + c, K.nTerms, p0, K.scale, margin) ? 1 : 0;
+                cFrac = frac_of(total, nBins);
+                ++nResolved;
             }
             // phaseC (:345-440)
             const float mRAn = (mRA - cur.meanFC) + mBackC;
@@ -1265,19 +1355,19 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
         return max(0, kLim - k0);
     };
     float* const spM = rowChunk;                                   // running mean after spectrum k
-    float* const spR = rowChunk + kStage;                          // running rms after k
-    float* const spS = rowChunk + 2 * kStage;                      // spectrumRMS pushed by k
-    float* const spB = rowChunk + 3 * kStage;                      // that value / history length
-    float* const spQ = rowChunk + 4 * kStage;                      // offset step of k
-    int* const spD = reinterpret_cast<int*>(rowChunk + 5 * kStage); // k moves the offset
-    float* const spP = rowChunk + 6 * kStage;                      // offset before k
-    float* const spMBC = rowChunk + 7 * kStage;                    // newest mean entry before k / history
-    float* const spRBC = rowChunk + 8 * kStage;                    // newest rms entry before k / history
-    float* const spF = rowChunk + 9 * kStage;                      // bad-channel fraction after k
-    float* const spMB = rowChunk + 10 * kStage;                    // newest mean-ring entry before k
-    float* const spRB = rowChunk + 11 * kStage;                    // newest rms-ring entry before k
-    static_assert(12 * kStage <= kRowChunk, "speculation arrays alias the row chunk");
-    __shared__ int sh_fail, sh_nrej, sh_nres, sh_still;
+    float* const spR = rowChunk + (kStage + kStagePad);                          // running rms after k
+    float* const spS = rowChunk + 2 * (kStage + kStagePad);                      // spectrumRMS pushed by k
+    float* const spB = rowChunk + 3 * (kStage + kStagePad);                      // that value / history length
+    float* const spQ = rowChunk + 4 * (kStage + kStagePad);                      // offset step of k
+    int* const spD = reinterpret_cast<int*>(rowChunk + 5 * (kStage + kStagePad)); // k moves the offset
+    float* const spP = rowChunk + 6 * (kStage + kStagePad);                      // offset before k
+    float* const spMBC = rowChunk + 7 * (kStage + kStagePad);                    // newest mean entry before k / history
+    float* const spRBC = rowChunk + 8 * (kStage + kStagePad);                    // newest rms entry before k / history
+    float* const spF = rowChunk + 9 * (kStage + kStagePad);                      // bad-channel fraction after k
+    float* const spMB = rowChunk + 10 * (kStage + kStagePad);                    // newest mean-ring entry before k
+    float* const spRB = rowChunk + 11 * (kStage + kStagePad);                    // newest rms-ring entry before k
+    static_assert(12 * (kStage + kStagePad) <= kRowChunk, "speculation arrays alias the row chunk");
+    __shared__ int sh_fail, sh_nrej, sh_nres;
     __shared__ float sh_pEnd;
     // spectrumRMS of a steady spectrum whose running mean before it is mPrev
     // (:288-311), and that value over the history length, as the scalar run
@@ -1310,18 +1400,70 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
         const bool useMOR = K.useMeanOverRMS != 0;
         const float mOR = s.meanOverRMS;
         const double rcpMOR = 1.0 / (double)mOR;
-        // The folds read their inputs sixteen spectra at a time, ahead of the
-        // dependent adds, so that LDS latency is paid once per sixteen; from
-        // the first multiple of four on, four spectra per LDS access.
-        constexpr int B = 16;
-        auto ld4 = [](const float* a, int k) { return *reinterpret_cast<const float4*>(a + k); };
-        auto ld4i = [](const int* a, int k) { return *reinterpret_cast<const int4*>(a + k); };
-        auto st4 = [](float* a, int k, float x, float y, float z, float w) {
-            *reinterpret_cast<float4*>(a + k) = make_float4(x, y, z, w);
+        // The folds are chains of dependent adds in one lane, so nothing but
+        // the adds may stand in them: from the first multiple of four on they
+        // read sixteen spectra at a time, four per LDS access, ask for the
+        // next sixteen before the adds of these, and run past the end to a
+        // whole sixteen (the arrays have that room, what is written there is
+        // not read, and the result is read back from the last spectrum).
+        // 511 spectra: 6.2 us a fold, 27 cycles a spectrum with its two adds;
+        // with waits for LDS and a select per spectrum for an offset that
+        // does not move it was 6.5 and 9.8.
+        constexpr int B = kStagePad;
+        auto ld16 = [](float* r, const float* a, int k) {
+#pragma unroll
+            for (int j = 0; j < B; j += 4) {
+                const float4 x = *reinterpret_cast<const float4*>(a + k + j);
+                r[j] = x.x; r[j + 1] = x.y; r[j + 2] = x.z; r[j + 3] = x.w;
+            }
         };
+        // keeps the reads above it from being moved to where they are used
+        auto issued = []() { asm volatile("" ::: "memory"); };
+        // v = op(v, x[k], y[k]) over spectra k to end; out[k] is v after it,
+        // or (before) ahead of it.  Returns v after the last.
+        auto fold = [&](float v, const float* x, const float* y, float* out, int k, int end, auto before, auto op) {
+            auto step16 = [&](const float* a, const float* c) {
+                float o[B];
+#pragma unroll
+                for (int j = 0; j < B; ++j) {
+                    const float u = op(v, a[j], c[j]);
+                    o[j] = before.value ? v : u;
+                    v = u;
+                }
+#pragma unroll
+                for (int j = 0; j < B; j += 4)
+                    *reinterpret_cast<float4*>(out + k + j) = make_float4(o[j], o[j + 1], o[j + 2], o[j + 3]);
+                k += B;
+            };
+            for (; k < end && (k & 3); ++k) {
+                const float u = op(v, x[k], y[k]);
+                out[k] = before.value ? v : u;
+                v = u;
+            }
+            if (k >= end) return v;
+            float a0[B], c0[B], a1[B], c1[B];
+            ld16(a0, x, k);
+            ld16(c0, y, k);
+            for (;;) {
+                ld16(a1, x, min(k + B, kStage));
+                ld16(c1, y, min(k + B, kStage));
+                issued();
+                step16(a0, c0);
+                if (k >= end) break;
+                ld16(a0, x, min(k + B, kStage));
+                ld16(c0, y, min(k + B, kStage));
+                issued();
+                step16(a1, c1);
+                if (k >= end) break;
+            }
+            return before.value ? op(out[end - 1], x[end - 1], y[end - 1]) : out[end - 1];
+        };
+        constexpr std::integral_constant<bool, false> after{};
+        constexpr std::integral_constant<bool, true> ahead{};
+        auto opRun = [](float v, float front, float back) { return (v - front) + back; };
+        auto opAdd = [](float v, float x, float) { return v + x; };
         // the mean-ring entry each spectrum's update adds: the last kept
         // spectrum's mean before it, or the state's newest entry
-        if (tid == 0) sh_still = 0;
         {
             const int k = tid;
             if (k >= k0 && k < kEnd) {
@@ -1331,63 +1473,8 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
             }
         }
         __syncthreads();
-        // a two-lane fold: (v - front/cap) + back/cap per spectrum
-        auto fold2 = [&](float v, const float* fc, const float* bc, float* out) {
-            int k = k0;
-            for (; k < kEnd && (k & 3); ++k) {
-                v = (v - fc[k]) + bc[k];
-                out[k] = v;
-            }
-            for (; k + B <= kEnd; k += B) {
-                float a[B], c[B];
-#pragma unroll
-                for (int j = 0; j < B; j += 4) {
-                    const float4 x = ld4(fc, k + j), y = ld4(bc, k + j);
-                    a[j] = x.x; a[j + 1] = x.y; a[j + 2] = x.z; a[j + 3] = x.w;
-                    c[j] = y.x; c[j + 1] = y.y; c[j + 2] = y.z; c[j + 3] = y.w;
-                }
-#pragma unroll
-                for (int j = 0; j < B; ++j) {
-                    v = (v - a[j]) + c[j];
-                    a[j] = v;
-                }
-#pragma unroll
-                for (int j = 0; j < B; j += 4) st4(out, k + j, a[j], a[j + 1], a[j + 2], a[j + 3]);
-            }
-            for (; k < kEnd; ++k) {
-                v = (v - fc[k]) + bc[k];
-                out[k] = v;
-            }
-        };
-        if (tid == 0) {
-            fold2(s.meanRunAve, soaMeanFC, spMBC, spM);
-        } else if (tid == 64) {
-            float f = s.fractionBadChannels;
-            int k = k0;
-            for (; k < kEnd && (k & 3); ++k) {
-                f += soaFracInc[k];
-                spF[k] = f;
-            }
-            for (; k + B <= kEnd; k += B) {
-                float fi[B];
-#pragma unroll
-                for (int j = 0; j < B; j += 4) {
-                    const float4 a = ld4(soaFracInc, k + j);
-                    fi[j] = a.x; fi[j + 1] = a.y; fi[j + 2] = a.z; fi[j + 3] = a.w;
-                }
-#pragma unroll
-                for (int j = 0; j < B; ++j) {
-                    f += fi[j];
-                    fi[j] = f;
-                }
-#pragma unroll
-                for (int j = 0; j < B; j += 4) st4(spF, k + j, fi[j], fi[j + 1], fi[j + 2], fi[j + 3]);
-            }
-            for (; k < kEnd; ++k) {
-                f += soaFracInc[k];
-                spF[k] = f;
-            }
-        }
+        if (tid == 0) fold(s.meanRunAve, soaMeanFC, spMBC, spM, k0, kEnd, after, opRun);
+        else if (tid == 64) fold(s.fractionBadChannels, soaFracInc, soaFracInc, spF, k0, kEnd, after, opAdd);
         __syncthreads();
         {
             const int k = tid;
@@ -1415,7 +1502,7 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
                 const float bmPrev = k == k0 ? s.bpMean : spM[k - 1];
                 const float delta = spM[k] - bmPrev;
                 int d = 0;
-                float qd = 0.0f;
+                float qd = -0.0f;
                 if (fabsf(delta) > 0.0f) {
                     d = 1;
                     qd = (float)((double)delta * rcpScale);
@@ -1423,77 +1510,18 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
                 }
                 spQ[k] = qd;
                 spD[k] = d;
-                if (!d) sh_still = 1;
             }
         }
         __syncthreads();
         if (tid == 0) {
-            fold2(s.rmsRunAve, soaRmsFC, spRBC, spR);
-        } else if (tid == 64 && !sh_still) {
-            // the bandpass offset when every spectrum moves it: p + q
-            float p = s.params0;
-            int k = k0;
-            for (; k < kEnd && (k & 3); ++k) {
-                spP[k] = p;
-                p += spQ[k];
-            }
-            for (; k + B <= kEnd; k += B) {
-                float q[B];
-#pragma unroll
-                for (int j = 0; j < B; j += 4) {
-                    const float4 a = ld4(spQ, k + j);
-                    q[j] = a.x; q[j + 1] = a.y; q[j + 2] = a.z; q[j + 3] = a.w;
-                }
-#pragma unroll
-                for (int j = 0; j < B; ++j) {
-                    const float pn = p + q[j];
-                    q[j] = p;
-                    p = pn;
-                }
-#pragma unroll
-                for (int j = 0; j < B; j += 4) st4(spP, k + j, q[j], q[j + 1], q[j + 2], q[j + 3]);
-            }
-            for (; k < kEnd; ++k) {
-                spP[k] = p;
-                p += spQ[k];
-            }
-            sh_pEnd = p;
+            fold(s.rmsRunAve, soaRmsFC, spRBC, spR, k0, kEnd, after, opRun);
         } else if (tid == 64) {
-            // the bandpass offset: p + q where the running mean moved
-            float p = s.params0;
-            const int* const spDi = spD;
-            int k = k0;
-            for (; k < kEnd && (k & 3); ++k) {
-                spP[k] = p;
-                if (spDi[k]) p += spQ[k];
-            }
-            for (; k + B <= kEnd; k += B) {
-                float q[B], op[B];
-                int d[B];
-#pragma unroll
-                for (int j = 0; j < B; j += 4) {
-                    const float4 a = ld4(spQ, k + j);
-                    const int4 e = ld4i(spDi, k + j);
-                    q[j] = a.x; q[j + 1] = a.y; q[j + 2] = a.z; q[j + 3] = a.w;
-                    d[j] = e.x; d[j + 1] = e.y; d[j + 2] = e.z; d[j + 3] = e.w;
-                }
-                // a select, not a branch: one add and one select per spectrum
-#pragma unroll
-                for (int j = 0; j < B; ++j) {
-                    op[j] = p;
-                    const float pn = p + q[j];
-                    p = d[j] ? pn : p;
-                }
-#pragma unroll
-                for (int j = 0; j < B; j += 4) st4(spP, k + j, op[j], op[j + 1], op[j + 2], op[j + 3]);
-            }
-            for (; k < kEnd; ++k) {
-                spP[k] = p;
-                if (spDi[k]) p += spQ[k];
-            }
-            sh_pEnd = p;
+            // the bandpass offset: p + q, where q is -0 if the running mean
+            // did not move (p + -0 is p for every p)
+            sh_pEnd = fold(s.params0, spQ, spQ, spP, k0, kEnd, ahead, opAdd);
         } else if (tid == 128) {
             sh_fail = kEnd;
+            sh_refold = kEnd;
             sh_nrej = 0;
             sh_nres = 0;
         }
@@ -1526,9 +1554,35 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
                 }
                 if (!ok) atomicMin(&sh_fail, k);
             }
+            // the bad-channel fractions that were folded with the decisions
+            // of the stage-start state: those that differ at their own state
+            const int slot = tid / kUndMax, c = tid % kUndMax;
+            if ((tid & ~63) < sh_nMany * kUndMax) {  // uniform over the wave
+                bool kept = false;
+                int km = -1;
+                if (slot < sh_nMany) {
+                    km = us.k[slot];
+                    if (km < k0 || km >= kEnd) km = -1;
+                    if (km >= 0 && c < us.n[slot])
+                        kept = und_kept(us, tid, K.nTerms, spP[km], K.scale, K.crFactor * spR[km]);
+                }
+                const unsigned long long all = __ballot(kept);
+                if (km >= 0 && c == 0) {
+                    const int nk = __popcll((all >> (tid & 63)) & ((1ull << kUndMax) - 1));
+                    const float f = frac_of(us.nKept[slot] + nk, nBins);
+                    if (f != soaFracInc[km]) {
+                        soaFracInc[km] = f;
+                        atomicMin(&sh_refold, km);
+                    }
+                }
+            }
         }
         __syncthreads();
         const int kf = sh_fail;
+        if (tid == 64 && sh_refold < kf) {
+            const int kr = sh_refold;
+            fold(kr > k0 ? spF[kr - 1] : s.fractionBadChannels, soaFracInc, soaFracInc, spF, kr, kf, after, opAdd);
+        }
         {
             const int k = tid;
             if (k >= k0 && k < kf) {
@@ -1544,7 +1598,7 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
                 rmsBuf[(s.rmsStart + (k - k0)) % K.cap] = rej ? spRB[k] : spS[k];
                 meanBuf[(s.meanStart + (k - k0)) % K.cap] = rej ? spMB[k] : soaMean[k];
                 if (rej) atomicAdd(&sh_nrej, 1);
-                if (stg[k].flags & PRE_ONE) atomicAdd(&sh_nres, 1);
+                if (stg[k].flags & (PRE_ONE | PRE_MANY)) atomicAdd(&sh_nres, 1);
             }
         }
         __syncthreads();
@@ -1660,14 +1714,48 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
             stageBase = t;
             stageN = min(kStage, tEnd - t);
             const int nPre = bx.valid ? min(stageN, preN - (t - tStart)) : 0;
-            for (int k = tid; k < nPre; k += kWalkThreads) {
-                const PreRec r = pre[t - tStart + k];
+            PreRec r;
+            r.flags = 0;
+            if (tid < nPre) r = pre[t - tStart + tid];
+            // a slot for each spectrum with a few undecided channels, in order
+            const unsigned long long many = __ballot((r.flags & PRE_MANY) != 0);
+            if (lane == 0) waveN[wave] = __popcll(many);
+            __syncthreads();
+            int slot = __popcll(many & ((1ull << lane) - 1)), nMany = 0;
+            for (int w = 0; w < kWalkThreads / 64; ++w) {
+                if (w < wave) slot += waveN[w];
+                nMany += waveN[w];
+            }
+            if (tid == 0) sh_nMany = min(nMany, kUndSlots);
+            if (slot >= kUndSlots) r.flags &= ~PRE_MANY;
+            if (r.flags & PRE_MANY) us.k[slot] = tid;
+            __syncthreads();
+            nMany = min(nMany, kUndSlots);
+            if (tid / kUndMax < nMany) {
+                const UndRec& u = undRec[t - tStart + us.k[tid / kUndMax]];
+                const int c = tid % kUndMax, n = u.n;
+                if (c == 0) {
+                    us.n[tid / kUndMax] = n;
+                    us.nKept[tid / kUndMax] = u.nKept;
+                }
+                if (c < n) {
+                    const int bin = u.bin[c];
+                    us.val[tid] = u.val[c];
+                    us.killed[tid] = bin_killed(kill, bin) ? 1 : 0;
+                    for (int j = 0; j < K.nTerms; ++j) us.terms[j][tid] = terms[(size_t)j * nBins + bin];
+                }
+            }
+            __syncthreads();
+            const int k = tid;
+            int bu = k, buf = k, lk = -1;
+            if (k < nPre) {
                 const int fl = r.flags | (r.badBands >= 4 ? PRE_REJ : 0);
                 stg[k].mean = r.mean;
                 stg[k].fracInc = r.fracInc;
                 stg[k].badBands = r.badBands;
                 stg[k].flags = fl;
                 stg[k].meanC = r.mean / capf;
+                stg[k].slot = slot;
                 // the speculative block takes the record the one undecided
                 // channel's decision at the stage-start state predicts
                 bool useK = false;
@@ -1685,7 +1773,16 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
                 }
                 soaMean[k] = useK ? r.meanK : r.mean;
                 soaMeanC[k] = useK ? r.meanK / capf : stg[k].meanC;
-                soaFracInc[k] = useK ? r.fracIncK : r.fracInc;
+                float frac = useK ? r.fracIncK : r.fracInc;
+                if (fl & PRE_MANY) {
+                    // at the stage-start state; the block counts them again
+                    int total = us.nKept[slot];
+                    for (int c = 0; c < us.n[slot]; ++c)
+                        total += und_kept(us, slot * kUndMax + c, K.nTerms, s.params0, K.scale,
+                                          K.crFactor * s.rmsRunAve) ? 1 : 0;
+                    frac = frac_of(total, nBins);
+                }
+                soaFracInc[k] = frac;
                 // a spectrum the mask keeps is predicted rejected when its
                 // mean exceeds the tolerance at the stage-start state
                 // (:394-425): the speculative block then checks that it is
@@ -1694,43 +1791,44 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
                 const bool tolRej = !maskRej && soaMean[k] - s.meanRunAve > tolS;
                 if (tolRej) stg[k].flags |= PRE_TOLREJ;
                 soaRej[k] = (maskRej || tolRej) ? 1 : 0;
+                const bool unres = (fl & PRE_UND) && !(fl & (PRE_ONE | PRE_MANY));
+                bu = unres ? k : kStage;
+                buf = (unres || (fl & PRE_FILL)) ? k : kStage;
+                lk = (maskRej || tolRej) ? -1 : k;
             }
-            {
-                // suffix minima over the stage (one thread per entry) of the
-                // spectra neither the fast run nor a speculative block takes:
-                // undecided channels other than one (blkU), or those or a
-                // last-good fill (blkUF)
-                const int k = tid;
-                int bu = k, buf = k, lk = -1;
-                if (k < nPre) {
-                    const int fl = stg[k].flags;
-                    const bool unres = (fl & PRE_UND) && !(fl & PRE_ONE);
-                    bu = unres ? k : kStage;
-                    buf = (unres || (fl & PRE_FILL)) ? k : kStage;
-                    lk = soaRej[k] ? -1 : k;
+            // suffix minima over the stage (one thread per entry) of the
+            // spectra neither the fast run nor a speculative block takes:
+            // undecided channels that are not staged (blkU), or those or a
+            // last-good fill (blkUF); and the last spectrum before each entry
+            // that the mask keeps: within the wave by shuffles, then across
+            // the waves through LDS
+            int lkx = __shfl_up(lk, 1, 64);
+            if (lane == 0) lkx = -1;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const int u = __shfl_down(bu, off, 64), uf = __shfl_down(buf, off, 64), p = __shfl_up(lkx, off, 64);
+                if (lane + off < 64) {
+                    bu = min(bu, u);
+                    buf = min(buf, uf);
                 }
-                blkU[k] = bu;
-                blkUF[k] = buf;
-                lastKept[k] = lk;
-                __syncthreads();
-                // and the prefix maxima of the kept indices (inclusive here,
-                // shifted by one below)
-                for (int off = 1; off < kStage; off <<= 1) {
-                    if (k + off < kStage) {
-                        bu = min(bu, blkU[k + off]);
-                        buf = min(buf, blkUF[k + off]);
-                    }
-                    if (k >= off) lk = max(lk, lastKept[k - off]);
-                    __syncthreads();
-                    blkU[k] = bu;
-                    blkUF[k] = buf;
-                    lastKept[k] = lk;
-                    __syncthreads();
-                }
-                lk = k > 0 ? lastKept[k - 1] : -1;
-                __syncthreads();
-                lastKept[k] = lk;
+                if (lane >= off) lkx = max(lkx, p);
             }
+            if (lane == 0) {
+                waveMin[0][wave] = bu;
+                waveMin[1][wave] = buf;
+            }
+            if (lane == 63) waveMax[wave] = max(lkx, lk);
+            __syncthreads();
+            for (int w = 0; w < kWalkThreads / 64; ++w) {
+                if (w > wave) {
+                    bu = min(bu, waveMin[0][w]);
+                    buf = min(buf, waveMin[1][w]);
+                }
+                if (w < wave) lkx = max(lkx, waveMax[w]);
+            }
+            blkU[k] = bu;
+            blkUF[k] = buf;
+            lastKept[k] = lkx;
             const int fv = s.rmsSize == K.cap && s.meanSize == K.cap && K.cap > kStage;
             if (fv) {
                 for (int k = tid; k < stageN; k += kWalkThreads) {
@@ -2275,6 +2373,7 @@ struct ppl_clipper {
     float2* d_stats = nullptr;
     SpecRec* d_rec = nullptr;
     PreRec* d_pre = nullptr;
+    UndRec* d_und = nullptr;
     LearnRec* d_learn = nullptr;
     Box* d_box = nullptr;
     float *d_bpLo = nullptr, *d_bpHi = nullptr, *d_lastGoodVer = nullptr;
@@ -2305,6 +2404,7 @@ void free_state(ppl_clipper* c)
     (void)hipFree(c->d_stats);
     (void)hipFree(c->d_rec);
     (void)hipFree(c->d_pre);
+    (void)hipFree(c->d_und);
     (void)hipFree(c->d_learn);
     (void)hipFree(c->d_box);
     (void)hipFree(c->d_bpLo);
@@ -2314,6 +2414,7 @@ void free_state(ppl_clipper* c)
     c->d_bs = nullptr;
     c->d_lastGoodVer = nullptr;
     c->d_pre = nullptr;
+    c->d_und = nullptr;
     c->d_learn = nullptr;
     c->d_box = nullptr;
     c->d_bpLo = c->d_bpHi = nullptr;
@@ -2529,14 +2630,17 @@ static int prepare(ppl_clipper* c, const ppl_clip_job& j)
     if ((int)j.nT > c->recCap) {
         (void)hipFree(c->d_rec);
         (void)hipFree(c->d_pre);
+        (void)hipFree(c->d_und);
         (void)hipFree(c->d_learn);
         (void)hipFree(c->d_stats);
         c->d_rec = nullptr;
         c->d_pre = nullptr;
+        c->d_und = nullptr;
         c->d_learn = nullptr;
         c->d_stats = nullptr;
         PPL_HIP(hipMalloc(&c->d_rec, sizeof(SpecRec) * j.nT));
         PPL_HIP(hipMalloc(&c->d_pre, sizeof(PreRec) * j.nT));     // a split run precomputes the whole run
+        PPL_HIP(hipMalloc(&c->d_und, sizeof(UndRec) * j.nT));
         PPL_HIP(hipMalloc(&c->d_learn, sizeof(LearnRec) * j.nT));
         PPL_HIP(hipMalloc(&c->d_stats, sizeof(float2) * j.nT));
         c->recCap = (int)j.nT;
@@ -2558,6 +2662,7 @@ static int prepare(ppl_clipper* c, const ppl_clip_job& j)
         h.kill = c->d_kill;
         h.box = c->d_box;
         h.pre = c->d_pre;
+        h.und = c->d_und;
         h.learn = c->d_learn;
         h.rec = c->d_rec;
         h.stats = c->d_stats;

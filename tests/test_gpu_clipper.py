@@ -179,6 +179,51 @@ def test_split_run_equals_run(orc, ppl):
     b.run_back()
 
 
+@pytest.mark.parametrize("n_und,every", [(2, 40), (16, 40), (17, 40), (5, 9)])
+def test_clipper_rejected_with_undecided_channels(orc, ppl, n_und, every):
+    """Every 40th (9th) spectrum loses half its channels to interference, so
+    it is rejected whatever n_und further channels do that lie within 2e-4 of
+    the channel threshold.  Up to 16 such channels are counted in the walk's
+    speculative blocks, for up to 32 spectra a stage of 512; more go to the
+    workgroup.  Outputs, flags and state are the oracle's bit for bit."""
+    n_sub, n_ch, n_t = 8, 16, 3000
+    x = _stream(1500 + n_t, n_sub, n_ch, seed=60 + n_und)
+    bp = _bp(n_sub, n_ch)
+    oc = orc.Clipper(bp, 10.0, 4.0, 1000, True)
+    gc = ppl.Clipper(bp, 10.0, 4.0, 1000, True)
+
+    def both(chunk):
+        ref = chunk.copy()
+        oc.run(ref)
+        d = torch.from_numpy(chunk).cuda()
+        gc.run(d)
+        assert np.array_equal(gc.flags(chunk.shape[0]), oc.last_flags(chunk.shape[0])[0])
+        assert np.array_equal(d.cpu().numpy(), ref, equal_nan=True)
+        st_o, _ = oc.state()
+        assert (np.float32(gc.stats()[0]), np.float32(gc.stats()[1])) == (st_o[0], st_o[1])
+
+    both(np.ascontiguousarray(x[:1500]))
+    before = gc.counters()
+    vals = gc.model(n_sub * n_ch)[3]
+    rng = np.random.default_rng(n_und)
+    y = np.ascontiguousarray(x[1500:])
+    flat = y.reshape(n_t, n_sub * n_ch)
+    for t in range(5, n_t, every):
+        bins = rng.permutation(n_sub * n_ch)
+        flat[t, bins[:64]] *= 50.0
+        near = bins[64:64 + n_und]
+        flat[t, near] = vals[near] + 10.0 * gc.stats()[1] * (1.0 + rng.uniform(-2e-4, 2e-4, n_und))
+    both(y)
+    after = gc.counters()
+    hit = len(range(5, n_t, every))
+    took = {k: after[k] - before[k] for k in after}
+    # (the noise itself adds spectra of both kinds)
+    if n_und > 16 or every < 10:
+        assert took["undecided"] > hit // 4, took
+    if n_und <= 16:
+        assert took["resolved"] > hit // 4, took
+
+
 def test_clipper_batch_equals_separate_runs(orc, ppl):
     """Beams of different shapes and spectrum counts in one batched run give
     the same outputs, flags and running statistics as separate runs, through
