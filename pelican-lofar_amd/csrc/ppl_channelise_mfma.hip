@@ -12,11 +12,14 @@
 //   Y[k2 + 16 k1] = sum_n1 G'[n1][k2] W_R^(n1 k1)         (stage 2)
 //
 // Stage 1 is a real GEMM [rows = (block, n1)] x [K = 32: Re, Im of 16 n2] x
-// [32: Re, Im of 16 k2] in v_mfma_f32_16x16x16 tiles.  Stage 2 is a 4-point
-// DFT in registers for R = 4 (a lane holds the four n1 of one block), and a
-// second MFMA GEMM for R = 16: the accumulator layout of a 16x16x16 MFMA
-// (lane l: column l % 16, rows 4 (l / 16) .. +3) is the B-operand layout of
-// the next one, so G' feeds stage 2 without leaving the registers.
+// [32: Re, Im of 16 k2] in v_mfma_f32_16x16x32 tiles, one instruction over
+// Re and Im together: an operand's slot (lane group g, element i) holds Re
+// n2 = 4 g + i for i < 4 and Im n2 = 4 g + i - 4 above, on both sides alike.
+// Stage 2 is a 4-point DFT in registers for R = 4 (a lane holds the four n1
+// of one block), and a second MFMA GEMM for R = 16: the accumulator of a
+// 16x16 MFMA (lane l: column l % 16, rows 4 (l / 16) .. +3) has a lane's Re
+// and Im of n1 = 4 g + i in those same slots, so G' feeds stage 2 without
+// leaving the registers, and both stages take one set of DFT constants.
 //
 // Precision (each product a*b of FP32 values):
 //   BF16x3: a = ah + al, b = bh + bl in bfloat16 (ah = RN(a), al = RN(a - ah));
@@ -28,6 +31,15 @@
 // 1.4e-4); the FP32 method: 6e-7.
 // Stokes-I (StokesGenerator.cpp:93-99) and the time integration
 // (StokesIntegrator.cpp:97-114) follow in FP32 in the reference's order.
+//
+// What bounds it is vector issue: of 47 subbands x 256 channels x 8192 blocks
+// (0.89 GB in and out) the BF16x3 form takes 295 us, 244 of them the issue of
+// 141 million wave instructions, 18 of 46 per sample the FIR and its
+// unpacking, and the matrix cores are busy a quarter of the time.  It was
+// 400 us with 16x16x16 tiles (twice the matrix time), one value rounded to
+// bfloat16 at a time, MFMA results copied from accumulation registers, loads
+// not asked for ahead of the DFT, and each polarisation's powers passed
+// through LDS behind barriers of its own.
 #include "ppl_internal.h"
 #include "ppl_ppf_batch.h"
 
@@ -44,11 +56,14 @@ namespace {
 
 using namespace ppl;
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kThreads = 256;
+// A thread filters two channels of 256, or one of 64.
+template <int N> constexpr int threads() { return N == 256 ? 256 : 128; }
 // blocks per tile: 16, and 8 at 256 channels so that four workgroups share a
 // CU's LDS (the filtered tile and the per-block Stokes-I take 40 KB)
 template <int N> constexpr int tile_blocks() { return N == 256 ? 8 : 16; }
@@ -57,39 +72,39 @@ struct C2 {
     float re, im;
 };
 
-// One operand fragment (four values of a 16x16x16 MFMA operand) in the
-// split precision PREC: hi and lo parts (lo unused by the rounded-once side).
+// One operand (eight values: Re and Im of four) in the split precision PREC:
+// hi and lo parts (lo unused by the rounded-once side).
 template <int PREC> struct Frag;
 template <> struct Frag<PPL_DFT_BF16X3> {
-    s16x4 hi, lo;
+    b16x8 hi, lo;
 };
 template <> struct Frag<PPL_DFT_FP16X2> {
-    h16x4 hi, lo;
+    h16x8 hi, lo;
 };
 
-__device__ __forceinline__ short bf16_bits(float x)
-{
-    const __bf16 b = (__bf16)x;  // round to nearest even
-    return __builtin_bit_cast(short, b);
-}
-__device__ __forceinline__ float bf16_val(short s) { return (float)__builtin_bit_cast(__bf16, s); }
-
-// Split four FP32 values (scale: exact power of two applied first, FP16 only).
+// Split four complex FP32 values.  Two values at a time are rounded to
+// bfloat16 by one instruction.
 template <int PREC>
-__device__ __forceinline__ Frag<PREC> split4(const float (&v)[4], float scale)
+__device__ __forceinline__ Frag<PREC> split(const float (&re)[4], const float (&im)[4])
 {
     Frag<PREC> f;
     if constexpr (PREC == PPL_DFT_BF16X3) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const short h = bf16_bits(v[i]);
-            f.hi[i] = h;
-            f.lo[i] = bf16_bits(v[i] - bf16_val(h));
+        for (int i = 0; i < 8; i += 2) {
+            const f32x2 v = i < 4 ? f32x2{re[i], re[i + 1]} : f32x2{im[i - 4], im[i - 3]};
+            const b16x2 h = __builtin_convertvector(v, b16x2);  // round to nearest even
+            const uint32_t u = __builtin_bit_cast(uint32_t, h);
+            const f32x2 d = {v.x - __uint_as_float(u << 16), v.y - __uint_as_float(u & 0xffff0000u)};
+            const b16x2 l = __builtin_convertvector(d, b16x2);
+            f.hi[i] = h.x;
+            f.hi[i + 1] = h.y;
+            f.lo[i] = l.x;
+            f.lo[i + 1] = l.y;
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float x = v[i] * scale;
+        for (int i = 0; i < 8; ++i) {
+            const float x = i < 4 ? re[i & 3] : im[i & 3];
             const _Float16 h = (_Float16)x;
             f.hi[i] = h;
             f.lo[i] = (_Float16)(x - (float)h);
@@ -98,32 +113,22 @@ __device__ __forceinline__ Frag<PREC> split4(const float (&v)[4], float scale)
     return f;
 }
 
-// acc += a * b in split precision; b is the constant (DFT matrix) side.
-template <int PREC>
-__device__ __forceinline__ f32x4 mma(const Frag<PREC>& a, const Frag<PREC>& b, f32x4 acc)
+// d * c (DFT constants) in split precision, FP32 accumulation; kData: which
+// side of the product the data is on.
+enum { kDataA, kDataB };
+template <int PREC, int SIDE>
+__device__ __forceinline__ f32x4 mma(const Frag<PREC>& d, const Frag<PREC>& c)
 {
-    if constexpr (PREC == PPL_DFT_BF16X3) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.lo, b.hi, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.hi, b.lo, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.hi, b.hi, acc, 0, 0, 0);
-    } else {
-        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(a.lo, b.hi, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(a.hi, b.hi, acc, 0, 0, 0);
-    }
-    return acc;
-}
-// The same with the data on the B side (stage 2: A = DFT matrix).
-template <int PREC>
-__device__ __forceinline__ f32x4 mma_b(const Frag<PREC>& a, const Frag<PREC>& b, f32x4 acc)
-{
-    if constexpr (PREC == PPL_DFT_BF16X3) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.lo, b.hi, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.hi, b.lo, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.hi, b.hi, acc, 0, 0, 0);
-    } else {
-        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(a.hi, b.lo, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(a.hi, b.hi, acc, 0, 0, 0);
-    }
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto one = [&](const auto& x, const auto& y) {
+        const auto& a = SIDE == kDataA ? x : y;
+        const auto& b = SIDE == kDataA ? y : x;
+        if constexpr (PREC == PPL_DFT_BF16X3) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+        else acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc, 0, 0, 0);
+    };
+    one(d.lo, c.hi);
+    if constexpr (PREC == PPL_DFT_BF16X3) one(d.hi, c.lo);
+    one(d.hi, c.hi);
     return acc;
 }
 
@@ -148,17 +153,23 @@ __device__ __forceinline__ void ppf_mfma_group(const uint32_t* __restrict__ in, 
     static_assert(R == 4 || R == 16, "split-precision DFT: 64 or 256 channels");
     constexpr int kTB = tile_blocks<N>();
     constexpr int H = TAPS - 1;
-    constexpr int ITEMS = (2 * N + kThreads - 1) / kThreads;  // (pol, channel) streams per thread
+    constexpr int kThreads = threads<N>();
+    constexpr int ITEMS = 2 * N / kThreads;  // (pol, channel) streams per thread
     constexpr int ROWT = kTB * R / 16;                        // 16-row tiles per polarisation
-    // Scales applied before the FP16 split and removed after each stage (exact
-    // powers of two).  |filtered sample| <= 32768 * sum_t |h| <= 8192 for the
-    // coefficients of PolyphaseCoefficients (peak 1/nCh, at most 16 taps) and
-    // |stage-1 output| <= 16 times that, so both stay inside binary16 unscaled,
-    // and unscaled noise keeps the low parts out of the subnormal range.
-    constexpr float kS1 = 1.0f;
-    constexpr float kS2 = 1.0f;
-    __shared__ float2 F[2][kTB][N];   // filtered blocks
-    __shared__ float P[kTB][N];       // Stokes-I per block (OUT 0)
+    // The FP16 split takes the values unscaled: |filtered sample| <= 32768 *
+    // sum_t |h| <= 8192 for the coefficients of PolyphaseCoefficients (peak
+    // 1/nCh, at most 16 taps) and |stage-1 output| <= 16 times that, so both
+    // stay inside binary16, and unscaled noise keeps the low parts out of the
+    // subnormal range.
+    // A stage-1 operand reads 16 channels of one block (R = 16), or 4 of each
+    // of 4 blocks, which the longer rows keep on different banks.
+    constexpr int kRowF = R == 4 ? N + 4 : N;
+    constexpr int kRowP = R == 4 ? N + 16 : N;
+    __shared__ float2 F[2][kTB][kRowF];  // filtered blocks
+    __shared__ float P[kTB][kRowP];      // Stokes-I per block (OUT 0)
+    // column of channel k in a row of P: R = 16 swaps sixteens so that a
+    // wave's four groups write on both halves of the banks
+    auto pcol = [](int k) { return R == 16 ? k ^ ((k >> 2) & 16) : k; };
 
     const int sub = group / nRuns;
     const int run = group % nRuns;
@@ -173,22 +184,18 @@ __device__ __forceinline__ void ppf_mfma_group(const uint32_t* __restrict__ in, 
     float hc[ITEMS][TAPS];
 #pragma unroll
     for (int q = 0; q < ITEMS; ++q) {
-        const int it = tid + kThreads * q;
-        const bool on = it < 2 * N;
-        const int pol = on ? it / N : 0, n = on ? it % N : 0;
+        const int it = tid + kThreads * q, pol = it / N, n = it % N;
         const uint32_t* x = in + (long)(2 * sub + pol) * T;
         const uint32_t* h = hist + (long)(2 * sub + pol) * H * N;
 #pragma unroll
         for (int t = 0; t < TAPS; ++t) {
-            hc[q][t] = on ? coeffs[t * N + n] : 0.0f;
+            hc[q][t] = coeffs[t * N + n];
             w[q][t] = {0.f, 0.f};
         }
 #pragma unroll
         for (int t = 0; t < H; ++t) {
             const long b = b0 - H + t;
-            C2 a = {0.f, 0.f};
-            if (on) a = b >= 0 ? load_c(x, b * N + n) : load_c(h, (long)(H + b) * N + n);
-            w[q][t + 1] = a;
+            w[q][t + 1] = b >= 0 ? load_c(x, b * N + n) : load_c(h, (long)(H + b) * N + n);
         }
     }
 
@@ -198,8 +205,10 @@ __device__ __forceinline__ void ppf_mfma_group(const uint32_t* __restrict__ in, 
         m &= N - 1;
         return {tw[2 * m], tw[2 * m + 1]};
     };
-    // stage 1 B operands: rows n2 = 4 grp + v, column k2 = col of W16
-    Frag<PREC> bR, bI, bNI;
+    // constants of the lane's slots: W16 at (4 grp + v, col), for the real and
+    // for the imaginary part of a product
+    Frag<PREC> cR, cI;
+    float twR[4], twI[4];  // W_N^(n1 k2) at k2 = col, n1 = the lane's rows
     {
         float r[4], i[4], ni[4];
 #pragma unroll
@@ -208,48 +217,44 @@ __device__ __forceinline__ void ppf_mfma_group(const uint32_t* __restrict__ in, 
             r[v] = c.re;
             i[v] = c.im;
             ni[v] = -c.im;
+            const C2 t = W(((4 * grp + v) % R) * col);
+            twR[v] = t.re;
+            twI[v] = t.im;
         }
-        bR = split4<PREC>(r, 1.0f);
-        bI = split4<PREC>(i, 1.0f);
-        bNI = split4<PREC>(ni, 1.0f);
-    }
-    // stage 2 A operands (R = 16): row k1 = col, columns n1 = 4 grp + v of W16
-    Frag<PREC> aR, aI, aNI;
-    if constexpr (R == 16) {
-        float r[4], i[4], ni[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const C2 c = W((col * (4 * grp + v)) * R);
-            r[v] = c.re;
-            i[v] = c.im;
-            ni[v] = -c.im;
-        }
-        aR = split4<PREC>(r, 1.0f);
-        aI = split4<PREC>(i, 1.0f);
-        aNI = split4<PREC>(ni, 1.0f);
+        cR = split<PREC>(r, ni);
+        cI = split<PREC>(i, r);
     }
 
-    for (int s0 = 0; s0 < len; s0 += kTB) {
-        const int nb = min(kTB, len - s0);
-        // ---- the tile's input, all loads in flight together
-        uint32_t xin[ITEMS][kTB];
+    // a tile's input, all loads in flight together; a tile's are asked for
+    // before the DFT of the one ahead of it
+    uint32_t xin[ITEMS][kTB];
+    auto load_tile = [&](int s0) {
+        const int nb = len - s0;
 #pragma unroll
         for (int q = 0; q < ITEMS; ++q) {
-            const int it = tid + kThreads * q;
-            const bool on = it < 2 * N;
-            const int pol = on ? it / N : 0, n = on ? it % N : 0;
+            const int it = tid + kThreads * q, pol = it / N, n = it % N;
             const uint32_t* x = in + (long)(2 * sub + pol) * T + (b0 + s0) * N + n;
+            if (nb >= kTB) {
 #pragma unroll
-            for (int s = 0; s < kTB; ++s) xin[q][s] = (on && s < nb) ? x[(long)s * N] : 0u;
+                for (int s = 0; s < kTB; ++s) xin[q][s] = x[s * N];
+            } else {
+#pragma unroll
+                for (int s = 0; s < kTB; ++s) xin[q][s] = s < nb ? x[s * N] : 0u;
+            }
         }
+    };
+    // Stokes-I rows of the tile, and their number in a whole one
+    const int nuTile = OUT == 0 ? kTB / integ : 0;
+    float* o0 = OUT == 0 ? out + ((b0 / integ) * nSub + sub) * (long)N : nullptr;
+    load_tile(0);
+    for (int s0 = 0; s0 < len; s0 += kTB) {
+        const int nb = min(kTB, len - s0);
         // ---- FIR of the tile's blocks into LDS
 #pragma unroll
         for (int s = 0; s < kTB; ++s) {
 #pragma unroll
             for (int q = 0; q < ITEMS; ++q) {
-                const int it = tid + kThreads * q;
-                const bool on = it < 2 * N;
-                const int pol = on ? it / N : 0, n = on ? it % N : 0;
+                const int it = tid + kThreads * q, pol = it / N, n = it % N;
 #pragma unroll
                 for (int t = 0; t < TAPS - 1; ++t) w[q][t] = w[q][t + 1];
                 const uint32_t xv = xin[q][s];
@@ -262,111 +267,102 @@ __device__ __forceinline__ void ppf_mfma_group(const uint32_t* __restrict__ in, 
                     f.re = f.re + cre;
                     f.im = f.im + cim;
                 }
-                if (on) F[pol][s][n] = make_float2(f.re, f.im);
+                F[pol][s][n] = make_float2(f.re, f.im);
+            }
+        }
+        if (s0 + kTB < len) load_tile(s0 + kTB);
+        __syncthreads();
+        // ---- DFT: a row tile's two polarisations in turn
+        for (int rt = wave; rt < ROWT; rt += kThreads / 64) {
+            float pw[4];
+#pragma unroll
+            for (int pol = 0; pol < 2; ++pol) {
+                // stage 1 operand: row (block, n1) = rt*16 + col, columns n2 = 4 grp + v
+                const int gr = rt * 16 + col;
+                const int sA = gr / R, n1A = gr % R;
+                float fr[4], fi[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float2 x = F[pol][sA][n1A + R * (4 * grp + v)];
+                    fr[v] = x.x;
+                    fi[v] = x.y;
+                }
+                const Frag<PREC> aF = split<PREC>(fr, fi);
+                const f32x4 gR = mma<PREC, kDataA>(aF, cR), gI = mma<PREC, kDataA>(aF, cI);
+                // G' = G W_N^(n1 k2): lane holds column k2 = col, rows rt*16 + 4 grp + v
+                float yr[4], yi[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+#pragma clang fp contract(fast)
+                    yr[v] = gR[v] * twR[v] - gI[v] * twI[v];
+                    yi[v] = gR[v] * twI[v] + gI[v] * twR[v];
+                }
+                int sOut;  // block of this lane's outputs
+                int kOut[4];
+                if constexpr (R == 4) {
+                    // rows 4 grp + v = (block grp, n1 = v): 4-point DFT over v in registers
+                    sOut = rt * 4 + grp;
+                    const C2 a0 = {yr[0], yi[0]}, a1 = {yr[1], yi[1]}, a2 = {yr[2], yi[2]}, a3 = {yr[3], yi[3]};
+                    const C2 s02 = {a0.re + a2.re, a0.im + a2.im}, d02 = {a0.re - a2.re, a0.im - a2.im};
+                    const C2 s13 = {a1.re + a3.re, a1.im + a3.im}, d13 = {a1.re - a3.re, a1.im - a3.im};
+                    yr[0] = s02.re + s13.re;
+                    yi[0] = s02.im + s13.im;
+                    yr[2] = s02.re - s13.re;
+                    yi[2] = s02.im - s13.im;
+                    yr[1] = d02.re + d13.im;  // X1 = d02 - i d13
+                    yi[1] = d02.im - d13.re;
+                    yr[3] = d02.re - d13.im;  // X3 = d02 + i d13
+                    yi[3] = d02.im + d13.re;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) kOut[v] = col + 16 * v;
+                } else {
+                    // stage 2 on the matrix cores: Y = W16 G' (rows k1, columns k2)
+                    sOut = rt;
+                    const Frag<PREC> bG = split<PREC>(yr, yi);
+                    const f32x4 oR = mma<PREC, kDataB>(bG, cR), oI = mma<PREC, kDataB>(bG, cI);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        yr[v] = oR[v];
+                        yi[v] = oI[v];
+                        kOut[v] = col + 16 * (4 * grp + v);
+                    }
+                }
+                if constexpr (OUT == 1) {
+                    if (sOut < nb) {
+                        const long b = b0 + s0 + sOut;
+                        float2* o = reinterpret_cast<float2*>(out) + ((b * nSub + sub) * 2 + pol) * (long)N;
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) o[kOut[v]] = make_float2(yr[v], yi[v]);
+                    }
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float p = yr[v] * yr[v] + yi[v] * yi[v];
+                        pw[v] = pol == 0 ? p : pw[v] + p;  // I = powerX + powerY
+                        if (pol == 1) P[sOut][pcol(kOut[v])] = pw[v];
+                    }
+                }
             }
         }
         __syncthreads();
-        // ---- DFT: row tiles of polarisation 0, then of polarisation 1
-        for (int pol = 0; pol < 2; ++pol) {
-        for (int rt = wave; rt < ROWT; rt += kThreads / 64) {
-            // stage 1 A operands: row (block, n1) = rt*16 + col, columns n2 = 4 grp + v
-            const int gr = rt * 16 + col;
-            const int sA = gr / R, n1A = gr % R;
-            float fr[4], fi[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float2 x = F[pol][sA][n1A + R * (4 * grp + v)];
-                fr[v] = x.x;
-                fi[v] = x.y;
-            }
-            const Frag<PREC> aFr = split4<PREC>(fr, kS1), aFi = split4<PREC>(fi, kS1);
-            f32x4 gR = {0.f, 0.f, 0.f, 0.f}, gI = {0.f, 0.f, 0.f, 0.f};
-            gR = mma<PREC>(aFr, bR, gR);
-            gR = mma<PREC>(aFi, bNI, gR);
-            gI = mma<PREC>(aFr, bI, gI);
-            gI = mma<PREC>(aFi, bR, gI);
-            // G' = G W_N^(n1 k2): lane holds column k2 = col, rows rt*16 + 4 grp + v
-            float yr[4], yi[4];
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = rt * 16 + 4 * grp + v;
-                const int n1 = row % R;
-                const C2 t = W(n1 * col);
-                const float a = gR[v] / kS1, c = gI[v] / kS1;
-                yr[v] = a * t.re - c * t.im;
-                yi[v] = a * t.im + c * t.re;
-            }
-            int sOut;  // block of this lane's outputs
-            int kOut[4];
-            if constexpr (R == 4) {
-                // rows 4 grp + v = (block grp, n1 = v): 4-point DFT over v in registers
-                sOut = rt * 4 + grp;
-                const C2 a0 = {yr[0], yi[0]}, a1 = {yr[1], yi[1]}, a2 = {yr[2], yi[2]}, a3 = {yr[3], yi[3]};
-                const C2 s02 = {a0.re + a2.re, a0.im + a2.im}, d02 = {a0.re - a2.re, a0.im - a2.im};
-                const C2 s13 = {a1.re + a3.re, a1.im + a3.im}, d13 = {a1.re - a3.re, a1.im - a3.im};
-                yr[0] = s02.re + s13.re;
-                yi[0] = s02.im + s13.im;
-                yr[2] = s02.re - s13.re;
-                yi[2] = s02.im - s13.im;
-                yr[1] = d02.re + d13.im;  // X1 = d02 - i d13
-                yi[1] = d02.im - d13.re;
-                yr[3] = d02.re - d13.im;  // X3 = d02 + i d13
-                yi[3] = d02.im + d13.re;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) kOut[v] = col + 16 * v;
-            } else {
-                // stage 2 on the matrix cores: Y = W16 G' (rows k1, columns k2)
-                sOut = rt;
-                const Frag<PREC> bGr = split4<PREC>(yr, kS2), bGi = split4<PREC>(yi, kS2);
-                f32x4 oR = {0.f, 0.f, 0.f, 0.f}, oI = {0.f, 0.f, 0.f, 0.f};
-                oR = mma_b<PREC>(aR, bGr, oR);
-                oR = mma_b<PREC>(aNI, bGi, oR);
-                oI = mma_b<PREC>(aI, bGr, oI);
-                oI = mma_b<PREC>(aR, bGi, oI);
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    yr[v] = oR[v] / kS2;
-                    yi[v] = oI[v] / kS2;
-                    kOut[v] = col + 16 * (4 * grp + v);
-                }
-            }
-            const bool live = sOut < nb;
-            if constexpr (OUT == 1) {
-                if (live) {
-                    const long b = b0 + s0 + sOut;
-                    float2* o = reinterpret_cast<float2*>(out) + ((b * nSub + sub) * 2 + pol) * (long)N;
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) o[kOut[v]] = make_float2(yr[v], yi[v]);
-                }
-            } else {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const float pw = yr[v] * yr[v] + yi[v] * yi[v];
-                    if (pol == 0) P[sOut][kOut[v]] = pw;
-                    else P[sOut][kOut[v]] = P[sOut][kOut[v]] + pw;  // I = powerX + powerY
-                }
-            }
-        }
-            __syncthreads();  // polarisation 0's powers are in P before polarisation 1 adds
-        }
         if constexpr (OUT == 0) {
-            __syncthreads();
             // integration over `integ` consecutive blocks, in time order
-            const int nu = nb / integ;
+            const int nu = nb == kTB ? nuTile : nb / integ;
             for (int e = tid; e < nu * N; e += kThreads) {
                 const int u = e / N, k = e % N;
                 float acc = 0.0f;
-                for (int j = 0; j < integ; ++j) acc = acc + P[u * integ + j][k];
-                const long ug = (b0 + s0) / integ + u;
-                out[(ug * nSub + sub) * (long)N + k] = acc;
+                for (int j = 0; j < integ; ++j) acc = acc + P[u * integ + j][pcol(k)];
+                o0[(long)u * nSub * N + k] = acc;
             }
+            o0 += (long)nuTile * nSub * N;
         }
-        __syncthreads();
+        // no wait here: the next tile writes F, last read ahead of the
+        // barrier above, and P only after its own first barrier
     }
 }
 
 template <int N, int TAPS, int PREC, int OUT>
-__global__ __launch_bounds__(kThreads) void ppf_mfma_kernel(const uint32_t* __restrict__ in,
+__global__ __launch_bounds__(threads<N>()) void ppf_mfma_kernel(const uint32_t* __restrict__ in,
                                                             const uint32_t* __restrict__ hist,
                                                             float* __restrict__ out,
                                                             const float* __restrict__ coeffs,
@@ -380,7 +376,7 @@ __global__ __launch_bounds__(kThreads) void ppf_mfma_kernel(const uint32_t* __re
 // Many plans' fused channeliser of one channel count, tap count and
 // precision in one launch: each workgroup finds its job in the table.
 template <int N, int TAPS, int PREC>
-__global__ __launch_bounds__(kThreads) void ppf_mfma_batch_kernel(const PPFBatch B)
+__global__ __launch_bounds__(threads<N>()) void ppf_mfma_batch_kernel(const PPFBatch B)
 {
     int local;
     const PPFJob& J = find_batch_job(B, local);
@@ -401,10 +397,10 @@ int launch(const ppl_ppf_config& c, const uint32_t* in, const uint32_t* hist, fl
         return PPL_E_ARG;
     }
     if (mode == 0)
-        hipLaunchKernelGGL((ppf_mfma_kernel<N, TAPS, PREC, 0>), dim3((unsigned)grid), dim3(kThreads), 0, st, in,
+        hipLaunchKernelGGL((ppf_mfma_kernel<N, TAPS, PREC, 0>), dim3((unsigned)grid), dim3(threads<N>()), 0, st, in,
                            hist, out, coeffs, tw, (int)c.nSub, nBlk, runLen, nRuns, (int)c.integrate);
     else
-        hipLaunchKernelGGL((ppf_mfma_kernel<N, TAPS, PREC, 1>), dim3((unsigned)grid), dim3(kThreads), 0, st, in,
+        hipLaunchKernelGGL((ppf_mfma_kernel<N, TAPS, PREC, 1>), dim3((unsigned)grid), dim3(threads<N>()), 0, st, in,
                            hist, out, coeffs, tw, (int)c.nSub, nBlk, runLen, nRuns, 1);
     PPL_LAUNCHED();
     return PPL_OK;
@@ -447,7 +443,7 @@ int launch_batch(PPFBatch& B, hipStream_t st)
             return PPL_E_ARG;
         }
     }
-    hipLaunchKernelGGL((ppf_mfma_batch_kernel<N, TAPS, PREC>), dim3((unsigned)blocks), dim3(kThreads), 0, st, B);
+    hipLaunchKernelGGL((ppf_mfma_batch_kernel<N, TAPS, PREC>), dim3((unsigned)blocks), dim3(threads<N>()), 0, st, B);
     PPL_LAUNCHED();
     return PPL_OK;
 }

@@ -55,6 +55,22 @@ def test_split_precision_history_and_fused_stokes(orc, ppl, prec):
     assert torch.equal(f, ref)
 
 
+@pytest.mark.parametrize("prec", ["bf16x3", "fp16x2"])
+@pytest.mark.parametrize("n_ch,n_blk,integ", [(64, 4, 4), (64, 36, 2), (64, 16, 16), (256, 2, 1), (256, 12, 4),
+                                              (256, 24, 8)])
+def test_split_precision_fused_stokes_tiles(orc, ppl, prec, n_ch, n_blk, integ):
+    """Whole, short and single tiles (16 blocks at 64 channels, 8 at 256) of
+    the fused form: the same bits as Stokes-I and integration of the spectra,
+    for both polarisations and every subband."""
+    n_sub = 3
+    h = orc.ppf_coefficients(8, n_ch, "kaiser").astype(np.float32)
+    xd = torch.from_numpy(noise_voltages(n_sub, n_blk * n_ch, 64.0, seed=n_ch + n_blk)).cuda()
+    spec = ppl.PPF(n_sub, n_ch, 8, h, precision=prec).spectra_i16(xd, n_blk)
+    f = ppl.PPF(n_sub, n_ch, 8, h, precision=prec, integrate=integ).stokes_i16(xd, n_blk)
+    st = ppl.stokes(spec, 1)
+    assert torch.equal(f, ppl.integrate(st, integ) if integ > 1 else st)
+
+
 def test_split_precision_rejects_shapes(ppl, orc):
     h = orc.ppf_coefficients(8, 128, "kaiser").astype(np.float32)
     with pytest.raises(ppl.PPLError):
