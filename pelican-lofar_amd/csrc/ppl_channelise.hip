@@ -14,7 +14,8 @@
 // instructions in this VALU-bound kernel.  Stokes-I and the integration keep
 // the reference's separate roundings.  The N-point forward DFT is a
 // Cooley-Tukey split N = R x G: an R-point DFT in registers, twiddles, then
-// a G-point radix-2 DIF FFT across lanes with xor shuffles.  Stokes-I
+// a G-point radix-2 DIF FFT across lanes, with xor shuffles for G < 64 and
+// two transforms at a time for G = 64 (pair_fft).  Stokes-I
 // (src/lib/src/StokesGenerator.cpp:93-99) and the integration over
 // `integrate` consecutive blocks (src/lib/src/StokesIntegrator.cpp:97-114)
 // are fused behind the FFT, so only int16 voltages are read and only the
@@ -116,6 +117,99 @@ __device__ __forceinline__ void lane_fft(float& re, float& im, const LaneTw& L)
     }
 }
 
+// Two 64-point FFTs at once, a's and b's, of the same arithmetic as lane_fft.
+// In lane_fft both lanes of a butterfly form one of its outputs each, and the
+// sum's lane multiplies by (1, 0).  Here the first two stages swap half of a
+// with half of b (v_permlane32_swap, v_permlane16_swap), so that a lane holds
+// both inputs of a butterfly and only differences are multiplied: 10
+// instructions a stage for both transforms where the lane form takes 12 and 4
+// LDS permutes.  The other four exchange within 16 lanes by DPP operands of
+// the multiply-add that forms the butterfly: sgn * pr + x, the butterfly's
+// output times sgn, which the twiddle takes back.  DPP has no xor by 4 but a
+// mirror of 8 lanes, xor by 7: lane l therefore holds sample fft_lane(l).
+// Lane l ends with bins k and k + 2 of a (l < 32) or b, k = pair_bin(l).
+// The kernel is bound by the issue of its instructions, 67 per sample with
+// the lane form: a 64-channel beam of 62 subbands and 32768 blocks takes 392
+// us instead of 445, 47 subbands of 256 channels and 8192 blocks 352 instead
+// of 406, the same bits.
+struct PairTw {
+    float r32, i32, r16, i16;         // twiddles of the first two stages' differences
+    float sgn[4], twr[3], twi[3];     // the others (m = 8, 4, 2, 1) as in LaneTw, the twiddles times sgn
+};
+__device__ __forceinline__ int fft_lane(int l) { return l ^ ((l & 4) ? 3 : 0); }
+__device__ __forceinline__ int pair_bin(int l)
+{
+    const int j = fft_lane(l);
+    return ((j >> 4) & 1) | ((j >> 1) & 4) | ((j << 1) & 8) | ((j << 3) & 16) | ((j << 5) & 32);
+}
+// The upper half of a for the lower half of b: of the wave, of each 32 lanes.
+__device__ __forceinline__ void swap32(float& a, float& b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float& a, float& b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void pair_stage(C2& a, C2& b, float twr, float twi)
+{
+    const C2 d = {a.re - b.re, a.im - b.im};
+    a = {a.re + b.re, a.im + b.im};
+    b = {__builtin_fmaf(d.re, twr, -(d.im * twi)), __builtin_fmaf(d.re, twi, d.im * twr)};
+}
+// x + sgn * (x of the lane that holds sample fft_lane(l) ^ M), in place, for
+// four values: one instruction each, where the compiler takes a move and a
+// multiply-add.  A DPP operand may not have been written by either of the
+// two instructions before: the wait covers the caller's, the four values'
+// order the rest.
+template <int M>
+__device__ __forceinline__ void row_butterfly(C2& a, C2& b, float sgn)
+{
+#define PPL_ROW_BUTTERFLY(CTRL)                                                   \
+    asm("s_nop 1\n\t"                                                             \
+        "v_fmac_f32_dpp %0, %0, %4 " CTRL " row_mask:0xf bank_mask:0xf\n\t"       \
+        "v_fmac_f32_dpp %1, %1, %4 " CTRL " row_mask:0xf bank_mask:0xf\n\t"       \
+        "v_fmac_f32_dpp %2, %2, %4 " CTRL " row_mask:0xf bank_mask:0xf\n\t"       \
+        "v_fmac_f32_dpp %3, %3, %4 " CTRL " row_mask:0xf bank_mask:0xf"           \
+        : "+v"(a.re), "+v"(a.im), "+v"(b.re), "+v"(b.im)                          \
+        : "v"(sgn))
+    if constexpr (M == 8) PPL_ROW_BUTTERFLY("row_ror:8");
+    else if constexpr (M == 4) PPL_ROW_BUTTERFLY("row_half_mirror");
+    else if constexpr (M == 2) PPL_ROW_BUTTERFLY("quad_perm:[2,3,0,1]");
+    else PPL_ROW_BUTTERFLY("quad_perm:[1,0,3,2]");
+#undef PPL_ROW_BUTTERFLY
+}
+template <int S, bool SPECTRA>
+__device__ __forceinline__ void row_fft(C2& a, C2& b, const PairTw& L)
+{
+    constexpr int m = 8 >> S;
+    row_butterfly<m>(a, b, L.sgn[S]);
+    if constexpr (m > 1) {
+        a = {__builtin_fmaf(a.re, L.twr[S], -(a.im * L.twi[S])), __builtin_fmaf(a.re, L.twi[S], a.im * L.twr[S])};
+        b = {__builtin_fmaf(b.re, L.twr[S], -(b.im * L.twi[S])), __builtin_fmaf(b.re, L.twi[S], b.im * L.twr[S])};
+        row_fft<S + 1, SPECTRA>(a, b, L);
+    } else if constexpr (SPECTRA) {
+        // a power does not see the last sgn
+        a = {a.re * L.sgn[S], a.im * L.sgn[S]};
+        b = {b.re * L.sgn[S], b.im * L.sgn[S]};
+    }
+}
+template <bool SPECTRA>
+__device__ __forceinline__ void pair_fft(C2& a, C2& b, const PairTw& L)
+{
+    swap32(a.re, b.re);
+    swap32(a.im, b.im);
+    pair_stage(a, b, L.r32, L.i32);
+    swap16(a.re, b.re);
+    swap16(a.im, b.im);
+    pair_stage(a, b, L.r16, L.i16);
+    row_fft<0, SPECTRA>(a, b, L);
+}
+
 template <int G>
 __device__ __forceinline__ int bitrev(int l)
 {
@@ -175,10 +269,10 @@ __device__ __forceinline__ void ppf_wave(const Tin* __restrict__ in, const typen
     constexpr int R = N / G;
     constexpr int RUNS_PER_WAVE = 64 / G;
     constexpr int H = TAPS - 1;
-    static_assert(!PS || (OUT == 0 && G == 64), "pol split: Stokes-I, one run per pair of waves");
+    static_assert(!PS || (OUT == 0 && G == 64 && R % 2 == 0), "pol split: Stokes-I, one run per pair of waves");
     const int lane = threadIdx.x & 63;
     const int grp = lane / G;
-    const int l = lane % G;
+    const int l = G == 64 ? fft_lane(lane) : lane % G;
     const int pol = PS ? (int)((threadIdx.x >> 6) & 1) : 0;  // the wave's polarisation (pol split)
     const long wavesPerSub = (nRuns + RUNS_PER_WAVE - 1) / RUNS_PER_WAVE;
     const int sub = (int)(waveId / wavesPerSub);
@@ -204,8 +298,27 @@ __device__ __forceinline__ void ppf_wave(const Tin* __restrict__ in, const typen
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int t = 0; t < TAPS; ++t) hc[r][t] = coeffs[t * N + l + G * r];
-    LaneTw ltw;
-    {
+    LaneTw ltw;   // G < 64
+    PairTw ptw;   // G = 64
+    if constexpr (G == 64) {
+        auto W = [&](int k) -> C2 { return {tw[2 * k], tw[2 * k + 1]}; };
+        const C2 a = W((l & 31) * R), b = W((l & 15) * 2 * R);
+        ptw.r32 = a.re;
+        ptw.i32 = a.im;
+        ptw.r16 = b.re;
+        ptw.i16 = b.im;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int m = 8 >> s;
+            const bool sumLane = (l & m) == 0;
+            ptw.sgn[s] = sumLane ? 1.0f : -1.0f;
+            if (m > 1) {
+                const C2 c = W((l & (m - 1)) * (N / (2 * m)));
+                ptw.twr[s] = sumLane ? 1.0f : -c.re;
+                ptw.twi[s] = sumLane ? 0.0f : -c.im;
+            }
+        }
+    } else {
         int s = 0;
 #pragma unroll
         for (int m = G / 2; m >= 1; m >>= 1, ++s) {
@@ -272,7 +385,17 @@ __device__ __forceinline__ void ppf_wave(const Tin* __restrict__ in, const typen
         };
         waveLen = max(steps(first), steps(first + 1));
     }
-    const int kLane = bitrev<G>(l);
+    // The transforms' outputs: bins kU of pair_fft's first and kU + 2 of its
+    // second value, for the polarisation (r, under pol split) of the half
+    const int half = lane >> 5;
+    const int kU = G == 64 ? pair_bin(lane) : 0;
+    // the channels of the Stokes-I sums this lane ends with
+    int kOut[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        kOut[r] = G < 64 ? bitrev<G>(l)
+                  : PS   ? (r & ~1) + half + R * (kU + 2 * (r & 1))
+                         : r + R * (kU + 2 * half);
     int inWindow = 0;  // blocks summed into the current integration window
     // output row of the current window: b0 is a multiple of integ (runLen is),
     // so row (b0 + s) / integ is counted instead of divided
@@ -338,17 +461,28 @@ __device__ __forceinline__ void ppf_wave(const Tin* __restrict__ in, const typen
             }
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                lane_fft<G>(f0[r].re, f0[r].im, ltw);
-                lane_fft<G>(f1[r].re, f1[r].im, ltw);
+                if constexpr (G < 64) {
+                    lane_fft<G>(f0[r].re, f0[r].im, ltw);
+                    lane_fft<G>(f1[r].re, f1[r].im, ltw);
+                } else if constexpr (!PS) {
+                    pair_fft<OUT == 1>(f0[r], f1[r], ptw);
+                } else if (r % 2 == 0) {
+                    pair_fft<false>(f0[r], f0[r | 1], ptw);
+                }
             }
             if constexpr (OUT == 1) {
                 if (live) {
 #pragma unroll
                     for (int r = 0; r < R; ++r) {
-                        const int k = r + R * kLane;
-                        float2* o = reinterpret_cast<float2*>(out) + ((long)(b * nSub + sub) * 2) * N + k;
-                        o[0] = make_float2(f0[r].re, f0[r].im);
-                        o[N] = make_float2(f1[r].re, f1[r].im);
+                        float2* o = reinterpret_cast<float2*>(out) + ((long)(b * nSub + sub) * 2) * N;
+                        if constexpr (G < 64) {
+                            o[kOut[r]] = make_float2(f0[r].re, f0[r].im);
+                            o[N + kOut[r]] = make_float2(f1[r].re, f1[r].im);
+                        } else {
+                            o += half * N + r + R * kU;
+                            o[0] = make_float2(f0[r].re, f0[r].im);
+                            o[2 * R] = make_float2(f1[r].re, f1[r].im);
+                        }
                     }
                 }
             } else if constexpr (PS) {
@@ -373,8 +507,7 @@ __device__ __forceinline__ void ppf_wave(const Tin* __restrict__ in, const typen
                     if (live && pol == 0) {
 #pragma unroll
                         for (int r = 0; r < R; ++r) {
-                            const int k = r + R * kLane;
-                            out[(uo * nSub + sub) * N + k] = acc[r];
+                            out[(uo * nSub + sub) * N + kOut[r]] = acc[r];
                         }
                     }
                     ++uo;
@@ -384,8 +517,10 @@ __device__ __forceinline__ void ppf_wave(const Tin* __restrict__ in, const typen
             } else {
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
-                    const float powerX = f0[r].re * f0[r].re + f0[r].im * f0[r].im;
-                    const float powerY = f1[r].re * f1[r].re + f1[r].im * f1[r].im;
+                    float powerX = f0[r].re * f0[r].re + f0[r].im * f0[r].im;
+                    float powerY = f1[r].re * f1[r].re + f1[r].im * f1[r].im;
+                    // two bins of one polarisation to one bin of both
+                    if constexpr (G == 64) swap32(powerX, powerY);
                     const float I = powerX + powerY;
                     acc[r] = acc[r] + I;
                 }
@@ -394,8 +529,7 @@ __device__ __forceinline__ void ppf_wave(const Tin* __restrict__ in, const typen
                     if (live) {
 #pragma unroll
                         for (int r = 0; r < R; ++r) {
-                            const int k = r + R * kLane;
-                            out[(uo * nSub + sub) * N + k] = acc[r];
+                            out[(uo * nSub + sub) * N + kOut[r]] = acc[r];
                         }
                     }
                     ++uo;

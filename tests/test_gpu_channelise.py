@@ -102,3 +102,28 @@ def test_fused_stokes_matches_stages(orc, ppl, n_ch, n_taps, n_sub, n_blk):
     err = np.max(np.abs(fused.cpu().numpy() - I64)) / np.mean(I64)
     assert torch.equal(fused, staged), (err, float((fused - staged).abs().max()))
     assert err < 1e-4, err
+
+
+@pytest.mark.parametrize("n_ch,n_taps", [(64, 4), (128, 8), (128, 16), (256, 4), (256, 16)])
+def test_tone_in_every_channel(orc, ppl, n_ch, n_taps):
+    """A tone at frequency k lands in its bin, in its own polarisation's
+    spectra only, for every k (the lane transform's order of bins and halves):
+    one subband per channel, the polarisation alternating."""
+    n_blk = 2 * n_taps
+    h = _coeffs(orc, n_taps, n_ch)
+    k = np.arange(n_ch)
+    t = np.arange(n_blk * n_ch)
+    z = 8000.0 * np.exp(2j * np.pi * np.outer(k, t % n_ch) / n_ch)
+    x = np.zeros((n_ch, 2, t.size, 2), np.int16)
+    x[k, k % 2, :, 0] = np.rint(z.real)
+    x[k, k % 2, :, 1] = np.rint(z.imag)
+    xd = torch.from_numpy(x).cuda()
+    spec = ppl.PPF(n_ch, n_ch, n_taps, h.astype(np.float32)).spectra_i16(xd, n_blk)
+    ref = orc.PPF(n_ch, 2, n_ch, n_taps, h).run_f64(x, n_blk)
+    got = spec.cpu().numpy()
+    got = got[..., 0] + 1j * got[..., 1].astype(np.float64)
+    assert np.max(np.abs(got - ref)) < 2e-5 * np.max(np.abs(ref))
+    fused = ppl.PPF(n_ch, n_ch, n_taps, h.astype(np.float32), integrate=2).stokes_i16(xd, n_blk)
+    assert torch.equal(fused, ppl.integrate(ppl.stokes(spec, 1), 2))
+    peak = fused[-1].reshape(n_ch, n_ch).argmax(dim=1).cpu().numpy()
+    assert np.array_equal(peak, (k + n_ch // 2) % n_ch)  # the filter puts frequency 0 in the middle
