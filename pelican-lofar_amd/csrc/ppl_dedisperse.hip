@@ -4,7 +4,13 @@
 // summed in channel order (the FP32 result is bit-identical to the
 // reference's per-thread channel loop, src/lib/DedispersionKernel.cu:32-43).
 //
-// Kernel shape.  One 256-thread workgroup owns a tile of TD = 4*ND DM trials
+// A plan without a tile of its own runs the register-window kernel (FP32 and
+// FP16, ppl_dedisp_window.h) or, from 128 tiles on, the u8 group kernel
+// (ppl_dedisp_u8group.h).  The kernels of this file run under a tile set by
+// the caller or the autotuner, for small u8 plans, where a plan's delays fit
+// no window, and behind the C seam.
+//
+// Their shape.  One 256-thread workgroup owns a tile of TD = 4*ND DM trials
 // by TT = 64*NT output samples.  Wave w of the workgroup accumulates ND DM
 // trials; lane l accumulates samples t0 + l + 64*i (i < NT), so every LDS
 // read of a wave is 64 consecutive words (bank-conflict free) and every
