@@ -12,19 +12,23 @@
 //   Y[k2 + 16 k1] = sum_n1 G'[n1][k2] W_R^(n1 k1)         (stage 2)
 //
 // Stage 1 is a real GEMM [rows = (block, n1)] x [K = 32: Re, Im of 16 n2] x
-// [32: Re, Im of 16 k2] in v_mfma_f32_16x16x32 tiles, one instruction over
-// Re and Im together: an operand's slot (lane group g, element i) holds Re
-// n2 = 4 g + i for i < 4 and Im n2 = 4 g + i - 4 above, on both sides alike.
-// Stage 2 is a 4-point DFT in registers for R = 4 (a lane holds the four n1
-// of one block), and a second MFMA GEMM for R = 16: the accumulator of a
-// 16x16 MFMA (lane l: column l % 16, rows 4 (l / 16) .. +3) has a lane's Re
-// and Im of n1 = 4 g + i in those same slots, so G' feeds stage 2 without
-// leaving the registers, and both stages take one set of DFT constants.
+// [32: Re, Im of 16 k2] in v_mfma_f32_16x16x16 tiles.  Stage 2 is a 4-point
+// DFT in registers for R = 4 (a lane holds the four n1 of one block), and a
+// second MFMA GEMM for R = 16: the accumulator layout of a 16x16x16 MFMA
+// (lane l: column l % 16, rows 4 (l / 16) .. +3) is the B-operand layout of
+// the next one, so G' feeds stage 2 without leaving the registers, and both
+// stages take one set of DFT constants.
+//
+// The sums' order is part of the results (an 8-bit buffer filled from them
+// changes with their last bits): Re then Im, the low parts before the high
+// ones, the twiddle's products rounded by themselves.  16x16x32 tiles over Re
+// and Im together and a fused twiddle take 295 us instead of 327 at the size
+// below and round otherwise.
 //
 // Precision (each product a*b of FP32 values):
 //   BF16x3: a = ah + al, b = bh + bl in bfloat16 (ah = RN(a), al = RN(a - ah));
 //           a*b ~ ah*bh + ah*bl + al*bh, three MFMAs, FP32 accumulation.
-//   FP16x2: the data split in binary16 (in range unscaled, see kS1), the DFT
+//   FP16x2: the data split in binary16 (in range unscaled, see ppf_mfma_group), the DFT
 //           matrices rounded once: a*b ~ (ah + al)*RN(b), two MFMAs.
 // Measured error against an all-FP64 chain, in units of the spectrum's RMS
 // (noise input): BF16x3 at most 2e-5 (RMS 4e-6), FP16x2 at most 7e-4 (RMS
@@ -33,13 +37,12 @@
 // (StokesIntegrator.cpp:97-114) follow in FP32 in the reference's order.
 //
 // What bounds it is vector issue: of 47 subbands x 256 channels x 8192 blocks
-// (0.89 GB in and out) the BF16x3 form takes 295 us, 244 of them the issue of
-// 141 million wave instructions, 18 of 46 per sample the FIR and its
-// unpacking, and the matrix cores are busy a quarter of the time.  It was
-// 400 us with 16x16x16 tiles (twice the matrix time), one value rounded to
-// bfloat16 at a time, MFMA results copied from accumulation registers, loads
-// not asked for ahead of the DFT, and each polarisation's powers passed
-// through LDS behind barriers of its own.
+// (0.89 GB in and out) the BF16x3 form takes 327 us, 270 of them the issue of
+// 156 million wave instructions, 18 of 51 per sample the FIR and its
+// unpacking, and the matrix cores are busy half the time.  It was 401 us with
+// one value rounded to bfloat16 at a time, MFMA results copied from
+// accumulation registers, loads not asked for ahead of the DFT, and each
+// polarisation's powers passed through LDS behind barriers of its own.
 #include "ppl_internal.h"
 #include "ppl_ppf_batch.h"
 
@@ -57,8 +60,8 @@ namespace {
 using namespace ppl;
 
 typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 b16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -72,63 +75,58 @@ struct C2 {
     float re, im;
 };
 
-// One operand (eight values: Re and Im of four) in the split precision PREC:
-// hi and lo parts (lo unused by the rounded-once side).
+// One operand fragment (four values of a 16x16x16 MFMA operand) in the
+// split precision PREC: hi and lo parts (lo unused by the rounded-once side).
 template <int PREC> struct Frag;
 template <> struct Frag<PPL_DFT_BF16X3> {
-    b16x8 hi, lo;
+    s16x4 hi, lo;
 };
 template <> struct Frag<PPL_DFT_FP16X2> {
-    h16x8 hi, lo;
+    h16x4 hi, lo;
 };
 
-// Split four complex FP32 values.  Two values at a time are rounded to
-// bfloat16 by one instruction.
+// Split four FP32 values.  Two at a time are rounded to bfloat16 by one
+// instruction.
 template <int PREC>
-__device__ __forceinline__ Frag<PREC> split(const float (&re)[4], const float (&im)[4])
+__device__ __forceinline__ Frag<PREC> split(const float (&x)[4])
 {
     Frag<PREC> f;
     if constexpr (PREC == PPL_DFT_BF16X3) {
-#pragma unroll
-        for (int i = 0; i < 8; i += 2) {
-            const f32x2 v = i < 4 ? f32x2{re[i], re[i + 1]} : f32x2{im[i - 4], im[i - 3]};
-            const b16x2 h = __builtin_convertvector(v, b16x2);  // round to nearest even
-            const uint32_t u = __builtin_bit_cast(uint32_t, h);
-            const f32x2 d = {v.x - __uint_as_float(u << 16), v.y - __uint_as_float(u & 0xffff0000u)};
-            const b16x2 l = __builtin_convertvector(d, b16x2);
-            f.hi[i] = h.x;
-            f.hi[i + 1] = h.y;
-            f.lo[i] = l.x;
-            f.lo[i + 1] = l.y;
-        }
+        uint2 hi, lo;
+        auto two = [](float a, float b, uint32_t& h, uint32_t& l) {
+            h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), b16x2));  // to nearest even
+            const f32x2 d = {a - __uint_as_float(h << 16), b - __uint_as_float(h & 0xffff0000u)};
+            l = __builtin_bit_cast(uint32_t, __builtin_convertvector(d, b16x2));
+        };
+        two(x[0], x[1], hi.x, lo.x);
+        two(x[2], x[3], hi.y, lo.y);
+        f.hi = __builtin_bit_cast(s16x4, hi);
+        f.lo = __builtin_bit_cast(s16x4, lo);
     } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float x = i < 4 ? re[i & 3] : im[i & 3];
-            const _Float16 h = (_Float16)x;
+        for (int i = 0; i < 4; ++i) {
+            const _Float16 h = (_Float16)x[i];
             f.hi[i] = h;
-            f.lo[i] = (_Float16)(x - (float)h);
+            f.lo[i] = (_Float16)(x[i] - (float)h);
         }
     }
     return f;
 }
 
-// d * c (DFT constants) in split precision, FP32 accumulation; kData: which
-// side of the product the data is on.
-enum { kDataA, kDataB };
-template <int PREC, int SIDE>
-__device__ __forceinline__ f32x4 mma(const Frag<PREC>& d, const Frag<PREC>& c)
+// acc += a * b in split precision, the data on side A (stage 1) or B (stage
+// 2): the low parts first, a's before b's.
+template <int PREC, bool DATA_A>
+__device__ __forceinline__ f32x4 mma(const Frag<PREC>& a, const Frag<PREC>& b, f32x4 acc)
 {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    auto one = [&](const auto& x, const auto& y) {
-        const auto& a = SIDE == kDataA ? x : y;
-        const auto& b = SIDE == kDataA ? y : x;
-        if constexpr (PREC == PPL_DFT_BF16X3) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-        else acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc, 0, 0, 0);
-    };
-    one(d.lo, c.hi);
-    if constexpr (PREC == PPL_DFT_BF16X3) one(d.hi, c.lo);
-    one(d.hi, c.hi);
+    if constexpr (PREC == PPL_DFT_BF16X3) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.lo, b.hi, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.hi, b.lo, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.hi, b.hi, acc, 0, 0, 0);
+    } else {
+        acc = DATA_A ? __builtin_amdgcn_mfma_f32_16x16x16f16(a.lo, b.hi, acc, 0, 0, 0)
+                     : __builtin_amdgcn_mfma_f32_16x16x16f16(a.hi, b.lo, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16f16(a.hi, b.hi, acc, 0, 0, 0);
+    }
     return acc;
 }
 
@@ -205,9 +203,8 @@ __device__ __forceinline__ void ppf_mfma_group(const uint32_t* __restrict__ in, 
         m &= N - 1;
         return {tw[2 * m], tw[2 * m + 1]};
     };
-    // constants of the lane's slots: W16 at (4 grp + v, col), for the real and
-    // for the imaginary part of a product
-    Frag<PREC> cR, cI;
+    // constants of the lane's slots: Re, Im and -Im of W16 at (4 grp + v, col)
+    Frag<PREC> cR, cI, cN;
     float twR[4], twI[4];  // W_N^(n1 k2) at k2 = col, n1 = the lane's rows
     {
         float r[4], i[4], ni[4];
@@ -221,8 +218,9 @@ __device__ __forceinline__ void ppf_mfma_group(const uint32_t* __restrict__ in, 
             twR[v] = t.re;
             twI[v] = t.im;
         }
-        cR = split<PREC>(r, ni);
-        cI = split<PREC>(i, r);
+        cR = split<PREC>(r);
+        cI = split<PREC>(i);
+        cN = split<PREC>(ni);
     }
 
     // a tile's input, all loads in flight together; a tile's are asked for
@@ -287,13 +285,16 @@ __device__ __forceinline__ void ppf_mfma_group(const uint32_t* __restrict__ in, 
                     fr[v] = x.x;
                     fi[v] = x.y;
                 }
-                const Frag<PREC> aF = split<PREC>(fr, fi);
-                const f32x4 gR = mma<PREC, kDataA>(aF, cR), gI = mma<PREC, kDataA>(aF, cI);
+                const Frag<PREC> aR = split<PREC>(fr), aI = split<PREC>(fi);
+                f32x4 gR = {0.f, 0.f, 0.f, 0.f}, gI = {0.f, 0.f, 0.f, 0.f};
+                gR = mma<PREC, true>(aR, cR, gR);
+                gI = mma<PREC, true>(aR, cI, gI);
+                gR = mma<PREC, true>(aI, cN, gR);
+                gI = mma<PREC, true>(aI, cR, gI);
                 // G' = G W_N^(n1 k2): lane holds column k2 = col, rows rt*16 + 4 grp + v
                 float yr[4], yi[4];
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-#pragma clang fp contract(fast)
                     yr[v] = gR[v] * twR[v] - gI[v] * twI[v];
                     yi[v] = gR[v] * twI[v] + gI[v] * twR[v];
                 }
@@ -318,8 +319,12 @@ __device__ __forceinline__ void ppf_mfma_group(const uint32_t* __restrict__ in, 
                 } else {
                     // stage 2 on the matrix cores: Y = W16 G' (rows k1, columns k2)
                     sOut = rt;
-                    const Frag<PREC> bG = split<PREC>(yr, yi);
-                    const f32x4 oR = mma<PREC, kDataB>(bG, cR), oI = mma<PREC, kDataB>(bG, cI);
+                    const Frag<PREC> bR = split<PREC>(yr), bI = split<PREC>(yi);
+                    f32x4 oR = {0.f, 0.f, 0.f, 0.f}, oI = {0.f, 0.f, 0.f, 0.f};
+                    oR = mma<PREC, false>(cR, bR, oR);
+                    oI = mma<PREC, false>(cI, bR, oI);
+                    oR = mma<PREC, false>(cN, bI, oR);
+                    oI = mma<PREC, false>(cR, bI, oI);
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
                         yr[v] = oR[v];

@@ -3,6 +3,8 @@ products, FP32 accumulation) against the oracle's FP64 DFT of the FP32 FIR and
 against the all-FP64 chain, with the error per output stated in units of the
 spectrum's RMS; history across calls, the fused Stokes-I/integration and the
 shapes it rejects."""
+import zlib
+
 import numpy as np
 import pytest
 import torch
@@ -69,6 +71,24 @@ def test_split_precision_fused_stokes_tiles(orc, ppl, prec, n_ch, n_blk, integ):
     f = ppl.PPF(n_sub, n_ch, 8, h, precision=prec, integrate=integ).stokes_i16(xd, n_blk)
     st = ppl.stokes(spec, 1)
     assert torch.equal(f, ppl.integrate(st, integ) if integ > 1 else st)
+
+
+# CRC32 of the spectra and of the x4 Stokes-I: the order in which the products
+# of the two stages are summed and rounded is part of the results
+SPLIT_BITS = {("bf16x3", 64): (684669127, 1842100593), ("bf16x3", 256): (938029680, 2424045220),
+              ("fp16x2", 64): (2888241824, 3139177054), ("fp16x2", 256): (1959157395, 4014488940)}
+
+
+@pytest.mark.parametrize("prec,n_ch", list(SPLIT_BITS))
+def test_split_precision_bits(ppl, prec, n_ch):
+    """The same bits from one version to the next (inputs and coefficients are
+    whole numbers over a power of two, so nothing else rounds)."""
+    n_sub, n_blk, rng = 3, 40, np.random.default_rng(n_ch)
+    h = (rng.integers(-4096, 4097, size=8 * n_ch) / (4096.0 * n_ch)).astype(np.float32)
+    xd = torch.from_numpy(rng.integers(-2000, 2001, size=(n_sub, 2, n_blk * n_ch, 2)).astype(np.int16)).cuda()
+    spec = ppl.PPF(n_sub, n_ch, 8, h, precision=prec).spectra_i16(xd, n_blk)
+    st = ppl.PPF(n_sub, n_ch, 8, h, precision=prec, integrate=4).stokes_i16(xd, n_blk)
+    assert tuple(zlib.crc32(t.cpu().numpy().tobytes()) for t in (spec, st)) == SPLIT_BITS[prec, n_ch]
 
 
 def test_split_precision_rejects_shapes(ppl, orc):
