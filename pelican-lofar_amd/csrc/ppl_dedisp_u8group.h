@@ -357,6 +357,13 @@ __global__ __launch_bounds__(64 * (kU8gSum + kU8gBuild)) void dedisperse_u8_grou
         add(a, 2);
         read(a, then, next.x & 0xffffu);
         add(b, 3);
+        // the sums so far are made before the barrier, so the reads of this
+        // pass's rows have landed when the builders overwrite them; those of
+        // the next pass may stay in flight
+#pragma unroll
+        for (int j = 0; j < kU8gND; ++j)
+            asm volatile("" : "+v"(acc[j][0]), "+v"(acc[j][1]), "+v"(acc[j][2]), "+v"(acc[j][3]), "+v"(acc[j][4]),
+                              "+v"(acc[j][5]), "+v"(acc[j][6]), "+v"(acc[j][7]));
         if ((p & 63) == 63) widen();
         bare_barrier();
         at = next, next = after;
