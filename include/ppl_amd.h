@@ -109,12 +109,25 @@ typedef struct {
  * beside it a tile for the others (input that is not 16-byte aligned, a tile
  * set later): the ring kernel at 32 trials x 512 samples (FP32, and u8 without
  * the group kernel) where a tile's delay spread fits its staged row, else the
- * one-word kernel at 32 (or fewer) trials x 512.  ppl_dedisp_info reports that tile.  Fails with PPL_E_CONFIG when nsampBuf <= maxshift
- * (the module's throw at :175-178), when dmStep < 0 (delays would decrease
- * with the trial index) or when a delayed read would leave the channel row. */
+ * one-word kernel at 32 (or fewer) trials x 512.  ppl_dedisp_info reports
+ * that tile, ppl_dedisp_plan_kernel the kernel.  Fails with PPL_E_CONFIG when
+ * nsampBuf <= maxshift (the module's throw at :175-178), when dmStep < 0
+ * (delays would decrease with the trial index) or when a delayed read would
+ * leave the channel row. */
 int ppl_dedisp_plan_create(ppl_dedisp_plan** plan, const ppl_dedisp_config* cfg);
 int ppl_dedisp_plan_destroy(ppl_dedisp_plan* plan);
 int ppl_dedisp_plan_info(const ppl_dedisp_plan* plan, ppl_dedisp_info* info);
+/* The kernel that ppl_dedisperse takes for input at d_in (null: any address
+ * that is a multiple of 16), and its DM x time tile.  staging: how the window
+ * kernel stages rows (0..2 split over the waves with 1, 2 or 4 pieces a lane,
+ * 3, 4 a row a wave with 2 or 4), 0 for the others. */
+enum { PPL_DD_ONE_WORD = 0, PPL_DD_RING = 1, PPL_DD_WINDOW = 2, PPL_DD_U8_GROUP = 3 };
+typedef struct {
+    int kernel;
+    int tileDM, tileT;
+    int staging;
+} ppl_dedisp_kernel_info;
+int ppl_dedisp_plan_kernel(const ppl_dedisp_plan* plan, const void* d_in, ppl_dedisp_kernel_info* info);
 /* Override the DM x time tile (the autotuner's hook); 0 keeps the default.  A
  * plan whose tile was set runs that tile and not the window or group kernel. */
 int ppl_dedisp_set_tile(ppl_dedisp_plan* plan, int tileDM, int tileT);

@@ -51,6 +51,13 @@ class DedispInfo(C.Structure):
                 ("fusedDelayDiffs", C.c_longlong)]
 
 
+class DedispKernelInfo(C.Structure):
+    _fields_ = [("kernel", C.c_int), ("tileDM", C.c_int), ("tileT", C.c_int), ("staging", C.c_int)]
+
+
+DEDISP_KERNELS = ("one_word", "ring", "window", "u8_group")
+
+
 class PPFConfig(C.Structure):
     _fields_ = [("nSub", C.c_uint), ("nPol", C.c_uint), ("nCh", C.c_uint), ("nTaps", C.c_uint),
                 ("coeffs", C.c_void_p), ("precision", C.c_int), ("integrate", C.c_uint)]
@@ -91,6 +98,7 @@ SIGNATURES = {
     "ppl_dedisp_plan_create": (i, [vp, vp]),
     "ppl_dedisp_plan_destroy": (i, [vp]),
     "ppl_dedisp_plan_info": (i, [vp, vp]),
+    "ppl_dedisp_plan_kernel": (i, [vp, vp, vp]),
     "ppl_dedisp_set_tile": (i, [vp, i, i]),
     "ppl_dedisp_set_shape": (i, [vp, i, i, i]),
     "ppl_dedisp_set_kernel": (i, [vp, i, i, i, i]),
@@ -240,6 +248,13 @@ class DedispPlan:
         info = DedispInfo()
         check(lib().ppl_dedisp_plan_info(self.h, C.byref(info)))
         self.tile = (info.tileDM, info.tileT, info.chanBlock, info.readBytes)
+
+    def kernel(self, d_in=None):
+        """(kernel name, tile DM trials, tile samples, staging) of a run on
+        d_in (None: any 16-byte aligned input); see ppl_dedisp_plan_kernel."""
+        info = DedispKernelInfo()
+        check(lib().ppl_dedisp_plan_kernel(self.h, None if d_in is None else _ptr(d_in), C.byref(info)))
+        return DEDISP_KERNELS[info.kernel], info.tileDM, info.tileT, info.staging
 
     def set_tile(self, tile_dm, tile_t, chan_block=0, read_bytes=4):
         """Tile (DM trials x samples), channels staged per block (0: as many

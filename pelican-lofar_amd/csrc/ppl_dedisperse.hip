@@ -1884,6 +1884,23 @@ extern "C" int ppl_dedisp_plan_info(const ppl_dedisp_plan* p, ppl_dedisp_info* i
     return PPL_OK;
 }
 
+extern "C" int ppl_dedisp_plan_kernel(const ppl_dedisp_plan* p, const void* d_in, ppl_dedisp_kernel_info* info)
+{
+    PPL_CHECK_ARG(p && info, "null argument");
+    info->staging = 0;
+    if (!p->ownTile && takes_table(ppl_dedisp_job{p, d_in, nullptr})) {
+        info->kernel = p->d_u8g ? PPL_DD_U8_GROUP : PPL_DD_WINDOW;
+        info->tileDM = p->d_u8g ? kU8gTD : kWinTD;
+        info->tileT = p->d_u8g ? kU8gTT : kWinShapes[p->winShape].TT;
+        if (p->d_win) info->staging = p->winStaging;
+        return PPL_OK;
+    }
+    info->kernel = p->rw == 16 ? PPL_DD_RING : PPL_DD_ONE_WORD;
+    info->tileDM = 4 * p->nd;
+    info->tileT = 64 * p->nt;
+    return PPL_OK;
+}
+
 extern "C" int ppl_dedisp_set_tile(ppl_dedisp_plan* p, int tileDM, int tileT)
 {
     return ppl_dedisp_set_kernel(p, tileDM, tileT, 0, 4);

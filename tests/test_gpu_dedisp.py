@@ -61,26 +61,42 @@ def test_f32_bit_exact_ragged(orc, ppl, shape, reads):
     assert np.array_equal(out, orc.dedisperse(x, d, p["nout"]))
 
 
-# (channels, trials, delay per trial in the last channel, output samples): the
-# register-window kernel's shapes and stagings, with remainders of trials,
-# samples, channels and rounds of channels at each
+# (channels, trials, delay per trial in the last channel, output samples) and,
+# for FP32 and FP16, the register-window kernel's tile and staging (None: the
+# delays fit no stage): every shape at every staging that a plan can take it
+# with, with remainders of trials, samples, channels and rounds of channels;
+# shared windows, windows of a trial's own, and both in one plan
 WINDOW_SHAPES = [
-    # long tiles (1280 samples; 1536 in FP16): one, two and four pieces a lane,
-    # shared windows, windows of a trial's own, and both in one plan
-    (7, 2113, 1.7, 5200), (18, 2113, 6.3, 5200), (3, 2113, 31.0, 5200), (2, 2113, 101.0, 5200),
-    # 768 samples: a row a wave, and split rows
-    (9, 1093, 5.9, 5100), (5, 1093, 23.0, 5100), (1, 1093, 90.0, 5100),
-    # 256 samples (512 in FP16): rows of two and four pieces, and split ones
-    (26, 37, 3.0, 700), (17, 37, 14.0, 700), (8, 37, 50.0, 700), (11, 33, 200.0, 700), (1, 1, 0.0, 224)]
+    # long tiles (1280 samples; 1536 in FP16)
+    ((7, 2113, 1.7, 5200), (1280, 0), (1536, 4)), ((18, 2113, 6.3, 5200), (1280, 0), (1536, 4)),
+    ((3, 2113, 31.0, 5200), (1280, 1), (1536, 0)), ((2, 2113, 101.0, 5200), (1280, 2), (1536, 1)),
+    ((2, 2113, 300.0, 5200), None, (1536, 2)), ((1, 1093, 90.0, 5100), (1280, 0), (1536, 4)),
+    # 768 samples
+    ((9, 1093, 5.9, 5500), (768, 4), (1536, 4)), ((5, 1093, 23.0, 5500), (768, 0), (1536, 0)),
+    ((3, 1093, 90.0, 5500), (768, 1), (1536, 1)), ((2, 1093, 200.0, 5500), (768, 2), (1536, 1)),
+    # 256 samples (512 in FP16)
+    ((9, 1093, 5.9, 5100), (256, 3), (1536, 4)), ((5, 1093, 23.0, 5100), (256, 4), (1536, 0)),
+    ((26, 37, 3.0, 700), (256, 3), (512, 3)), ((17, 37, 14.0, 700), (256, 4), (512, 3)),
+    ((7, 37, 30.0, 700), (256, 0), (512, 4)), ((8, 37, 50.0, 700), (256, 0), (512, 0)),
+    ((6, 37, 100.0, 700), (256, 1), (512, 0)), ((11, 33, 200.0, 700), (256, 2), (512, 1)),
+    ((3, 33, 400.0, 700), None, (512, 2)), ((1, 1, 0.0, 224), (256, 3), (512, 3))]
+
+
+def test_window_shapes_cover_every_kernel():
+    f32 = {k for _, k, _ in WINDOW_SHAPES if k}
+    f16 = {k for _, _, k in WINDOW_SHAPES if k}
+    assert f32 == {(1280, g) for g in (0, 1, 2)} | {(768, g) for g in (0, 1, 2, 4)} | {(256, g) for g in range(5)}
+    assert f16 == {(1536, g) for g in (0, 1, 2, 4)} | {(512, g) for g in range(5)}
 
 
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
-@pytest.mark.parametrize("n_chan,tdms,slope,n_out", WINDOW_SHAPES)
-def test_window_kernel_bit_exact(orc, ppl, dtype, n_chan, tdms, slope, n_out):
+@pytest.mark.parametrize("shape,f32,f16", WINDOW_SHAPES)
+def test_window_kernel_bit_exact(orc, ppl, dtype, shape, f32, f16):
     """Plans without a tile of their own, whose rows are whole 16-byte pieces:
     every sum equals the oracle's channel-order sum, infinities and NaN at
     the end of a row included; the same input 4 bytes off a 16-byte boundary
     (the one-word and ring kernels) gives the same."""
+    n_chan, tdms, slope, n_out = shape
     tsamp, fch1, foff = 0.00032768, 150.0, -0.05
     f = fch1 + foff * (n_chan - 1)
     shift = 4148.741601 * (1.0 / f / f - 1.0 / fch1 / fch1) if n_chan > 1 else 1.0
@@ -95,25 +111,33 @@ def test_window_kernel_bit_exact(orc, ppl, dtype, n_chan, tdms, slope, n_out):
     exp = orc.dedisperse(host, d, p["nout"])
     dev = torch.from_numpy(x if dtype == "f32" else host.view(np.float16)).cuda()
     plan = ppl.DedispPlan(**cfg, dtype=dtype)
+    want = f32 if dtype == "f32" else f16
+    name, tile_dm, tile_t, staging = plan.kernel(dev)
+    assert (name, tile_dm, (tile_t, staging)) == ("window", 32, want) if want else name == "one_word"
     assert np.array_equal(plan.run(dev).cpu().numpy(), exp, equal_nan=True)
     off = torch.empty(dev.numel() + 8, dtype=dev.dtype, device="cuda")[4 // dev.element_size():][:dev.numel()]
     off.copy_(dev.view(-1))
+    assert plan.kernel(off)[0] in ("ring", "one_word")
     assert np.array_equal(plan.run(off).cpu().numpy(), exp, equal_nan=True)
 
 
 # (channels, trials, samples of delay per trial in the last channel, output
 # samples) for the u8 group kernel, which takes 128 tiles of 48 trials x 1024
 # samples and more: ends of groups of four channels, of tiles and of the 64
-# passes between widenings; more passes than groups where the delays are steep;
-# the last with too many, which the ring kernel takes
-U8_GROUP_SHAPES = [(1, 3100, 0.0, 1030), (2, 5, 0.5, 130900), (3, 48, 1.0, 131200), (5, 49, 4.0, 65600),
-                   (53, 97, 6.3, 43100), (64, 150, 0.02, 33000), (258, 50, 2.0, 65600), (131, 96, 10.0, 65600),
-                   (6, 97, 9.9, 43100)]
+# passes between widenings, one pass a group and more
+U8_GROUP_SHAPES = [(1, 3100, 0.0, 1030), (2, 5, 0.01, 131100), (3, 48, 0.02, 131200), (4, 96, 0.03, 65700),
+                   (5, 49, 0.04, 65700), (6, 97, 0.05, 43800), (53, 97, 0.5, 43800), (53, 97, 1.0, 43800),
+                   (64, 150, 0.02, 33000), (131, 96, 1.2, 65700), (258, 50, 2.0, 65600), (514, 145, 5.2, 33000),
+                   (1030, 49, 10.3, 66000)]
+# steep delays: two passes a group and more, which the ring kernel takes
+U8_RING_SHAPES = [(2, 5, 0.5, 130900), (3, 48, 1.0, 131200), (5, 49, 4.0, 65600), (53, 97, 6.3, 43100),
+                  (131, 96, 10.0, 65600), (6, 97, 9.9, 43100)]
 
 
-@pytest.mark.parametrize("n_chan,tdms,slope,n_out", U8_GROUP_SHAPES)
+@pytest.mark.parametrize("kernel,n_chan,tdms,slope,n_out", [("u8_group", *r) for r in U8_GROUP_SHAPES] +
+                         [("ring", *r) for r in U8_RING_SHAPES])
 @pytest.mark.parametrize("full", [False, True])
-def test_u8_group_kernel_exact(orc, ppl, n_chan, tdms, slope, n_out, full):
+def test_u8_group_kernel_exact(orc, ppl, kernel, n_chan, tdms, slope, n_out, full):
     """u8 plans without a tile of their own: the oracle's sums, with every
     value at 255 too (the 16-bit partial sums at their largest), and the same
     from an input 4 bytes off a 16-byte boundary (the ring and one-word
@@ -133,9 +157,11 @@ def test_u8_group_kernel_exact(orc, ppl, n_chan, tdms, slope, n_out, full):
     exp = orc.dedisperse(x, d, p["nout"])
     dev = torch.from_numpy(x).cuda()
     plan = ppl.DedispPlan(**cfg, dtype="u8")
+    assert plan.kernel(dev)[0] == kernel
     assert np.array_equal(plan.run(dev).cpu().numpy(), exp)
     off = torch.empty(dev.numel() + 8, dtype=torch.uint8, device="cuda")[4:4 + dev.numel()]
     off.copy_(dev.view(-1))
+    assert plan.kernel(off)[0] == ("one_word" if kernel == "u8_group" else "ring")
     assert np.array_equal(plan.run(off).cpu().numpy(), exp)
 
 
@@ -266,11 +292,13 @@ def test_reference_c_seam_lofar_equals_plan(orc, ppl):
     del x, out, want
 
 
-def test_default_fp32_tile_is_the_ring_and_batches_fall_back(orc, ppl):
-    """An FP32 plan starts on the ring tile (32 x 512, 16-byte reads) where
-    its delay spread fits, and on one-sample reads where it does not; a batch
-    under job 0's own tile falls back to one-sample reads when another job's
-    spread does not fit the ring.  Every output equals the oracle's."""
+def test_default_fp32_kernel_and_set_ring_tile(orc, ppl):
+    """An FP32 plan runs the window kernel, beside a tile for other input: the
+    ring (32 x 512, 16-byte reads) where its delay spread fits, one-sample
+    reads where it does not.  A batch without a tile runs each plan so; under
+    job 0's ring tile, once set, it falls back to one-sample reads when another
+    job's spread does not fit the ring, and takes the window kernel again when
+    the tile is cleared.  Every output equals the oracle's."""
     wide = dict(SMALL, dm_step=300 / 128, nsamp_buf=16384, tdms=100)
     rng = np.random.default_rng(15)
     xs, exps, plans = [], [], []
@@ -279,13 +307,23 @@ def test_default_fp32_tile_is_the_ring_and_batches_fall_back(orc, ppl):
         p, d = _oracle(orc, x, cfg)
         plan = ppl.DedispPlan(**cfg)
         assert (plan.tile == (32, 512, 0, 16)) == ring, plan.tile
+        assert plan.kernel()[0] == "window"
         assert np.array_equal(plan.run(torch.from_numpy(x).cuda()).cpu().numpy(), orc.dedisperse(x, d, p["nout"]))
         xs.append(torch.from_numpy(x).cuda())
         exps.append(orc.dedisperse(x, d, p["nout"]))
         plans.append(plan)
-    outs = ppl.dedisperse_batch(plans, xs)
-    for o, e in zip(outs, exps):
-        assert np.array_equal(o.cpu().numpy(), e)
+
+    def check():
+        for o, e in zip(ppl.dedisperse_batch(plans, xs), exps):
+            assert np.array_equal(o.cpu().numpy(), e)
+
+    check()
+    plans[0].set_tile(32, 512, 0, 16)
+    assert plans[0].kernel() == ("ring", 32, 512, 0)
+    check()
+    plans[0].clear_tile()
+    assert plans[0].kernel()[0] == "window"
+    check()
 
 
 def test_plan_counts_fused_delay_differences(orc, ppl):
