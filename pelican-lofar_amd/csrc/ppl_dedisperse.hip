@@ -1692,8 +1692,10 @@ int window_table(ppl_dedisp_plan* p)
     const int nChan = (int)p->cfg.nChan, nsamp = (int)p->cfg.nsampBuf, elem = elem_bytes(p->cfg.dtype);
     int staging = 0;
     const int shape = window_shape(p->cfg.dtype, (int)p->cfg.tdms, p->nOut, span_of(p, kWinTD), &staging);
+    // Split rows step from one row's first byte to the next's in 32 bits: less
+    // than two rows.
     if (shape < 0 || (long)nsamp * elem % 16 != 0 || (long)p->nOut * elem % 16 != 0 ||
-        (long)nChan * nsamp >= (1L << 31))
+        (long)nChan * nsamp >= (1L << 31) || (!win_whole(staging) && 2L * nsamp * elem >= (1L << 32)))
         return PPL_OK;
     const int nDMTiles = ((int)p->cfg.tdms + kWinTD - 1) / kWinTD;
     const size_t bytes = win_table_bytes(nDMTiles, nChan);

@@ -121,6 +121,18 @@ def test_window_kernel_bit_exact(orc, ppl, dtype, shape, f32, f16):
     assert np.array_equal(plan.run(off).cpu().numpy(), exp, equal_nan=True)
 
 
+@pytest.mark.parametrize("nsamp,name", [(1 << 29, "ring"), ((1 << 29) - 224, "window"), (1000000000, "ring")])
+def test_window_kernel_refuses_rows_past_its_steps(ppl, nsamp, name):
+    """Two channels of up to 10^9 samples whose delays are 2e8 apart: split
+    rows step from a row's first byte to the next's in 32 bits, so from 2^29
+    FP32 samples on the plan keeps its tile (no data is needed to see it)."""
+    tsamp, fch1, foff = 0.00032768, 150.0, -0.05
+    f = fch1 + foff
+    shift = 4148.741601 * (1.0 / f / f - 1.0 / fch1 / fch1)
+    plan = ppl.DedispPlan(2, nsamp, 33, 2e8 * tsamp / shift, tsamp / shift, tsamp, fch1, foff)
+    assert plan.kernel()[0] == name, plan.kernel()
+
+
 # (channels, trials, samples of delay per trial in the last channel, output
 # samples) for the u8 group kernel, which takes 128 tiles of 48 trials x 1024
 # samples and more: ends of groups of four channels, of tiles and of the 64
