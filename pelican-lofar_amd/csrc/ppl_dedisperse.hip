@@ -1154,13 +1154,14 @@ __global__ void build_delays_kernel(const float* __restrict__ shift, int nChan, 
                                     int32_t* __restrict__ delayT)
 {
     const int dm = blockIdx.x * blockDim.x + threadIdx.x;
-    const int c = blockIdx.y;
-    if (dm >= tdmsPad || c >= nChan) return;
+    if (dm >= tdmsPad) return;
     const int d = dm < tdms ? dm : tdms - 1;
     const float prod = (float)d * mdmstep;
     const float dmval = mstartdm + prod;
-    const float p = shift[c] * dmval;
-    delayT[(size_t)c * tdmsPad + dm] = (int32_t)p;
+    for (int c = blockIdx.y; c < nChan; c += gridDim.y) {
+        const float p = shift[c] * dmval;
+        delayT[(size_t)c * tdmsPad + dm] = (int32_t)p;
+    }
 }
 
 // The FP32 ring kernel's table for DM tiles of TD trials, from a device delay
@@ -1644,20 +1645,29 @@ int tile_span(const std::vector<int32_t>& d, int tdms, int nChan, int TD)
     return span;
 }
 
-int upload_delays(ppl_dedisp_plan* p)
+// The plan's device delays, from its shifts as the host's (a transposed copy
+// of those, 32 MB for a LOFAR-size beam, took half of the plan's creation).
+int device_delays(ppl_dedisp_plan* p)
 {
     const int tdms = (int)p->cfg.tdms, nChan = (int)p->cfg.nChan;
     const int pad = ((tdms + 63) / 64) * 64;
-    std::vector<int32_t> t((size_t)nChan * pad);
-    for (int c = 0; c < nChan; ++c)
-        for (int dm = 0; dm < pad; ++dm)
-            t[(size_t)c * pad + dm] = p->delays[(size_t)std::min(dm, tdms - 1) * nChan + c];
-    if (p->d_delayT) PPL_HIP(hipFree(p->d_delayT));
-    p->d_delayT = nullptr;
-    PPL_HIP(hipMalloc(&p->d_delayT, t.size() * sizeof(int32_t)));
-    PPL_HIP(hipMemcpy(p->d_delayT, t.data(), t.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     p->tdmsPad = pad;
     for (int k = 0; k < 4; ++k) p->spanTD[k] = tile_span(p->delays, tdms, nChan, 8 << k);
+    PPL_HIP(hipMalloc(&p->d_delayT, (size_t)nChan * pad * sizeof(int32_t)));
+    float* d_shift = nullptr;
+    PPL_HIP(hipMalloc(&d_shift, nChan * sizeof(float)));
+    hipError_t e = hipMemcpy(d_shift, p->shift.data(), nChan * sizeof(float), hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(build_delays_kernel, dim3(cdiv(pad, 256), std::min(nChan, 65535)), dim3(256), 0, nullptr,
+                           d_shift, nChan, tdms, pad, p->mstartdm, p->mdmstep, p->d_delayT);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // the plan may be used on any stream
+    (void)hipFree(d_shift);
+    if (e != hipSuccess) {
+        set_error("dedispersion: device delays: %s", hipGetErrorString(e));
+        return PPL_E_HIP;
+    }
     return PPL_OK;
 }
 
@@ -1845,7 +1855,7 @@ extern "C" int ppl_dedisp_plan_create(ppl_dedisp_plan** plan, const ppl_dedisp_c
     p->defNd = p->nd;
     p->defNt = p->nt;
     p->defRw = p->rw;
-    int rc = upload_delays(p);
+    int rc = device_delays(p);
     if (rc == PPL_OK) rc = window_table(p);
     if (rc == PPL_OK) rc = u8_kernel(p);
     if (rc != PPL_OK) {

@@ -338,6 +338,23 @@ def test_default_fp32_kernel_and_set_ring_tile(orc, ppl):
     check()
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+def test_more_channels_than_a_grid_has_rows(orc, ppl, dtype):
+    """66001 channels: the plan's delays are made on the device by a grid of
+    at most 65535 rows of blocks."""
+    cfg = dict(n_chan=66001, nsamp_buf=512, tdms=5, dm_low=0.15, dm_step=0.25, tsamp=0.00032768, fch1=150.0, foff=-2e-4)
+    x = np.random.default_rng(9).normal(size=(cfg["n_chan"], cfg["nsamp_buf"])).astype(np.float32)
+    p, d = _oracle(orc, x, cfg)
+    assert d[-1, -1] > d[-1, 60000] > 40
+    host = x if dtype == "f32" else orc.f32_to_f16_bits(x)
+    dev = torch.from_numpy(x if dtype == "f32" else host.view(np.float16)).cuda()
+    plan = ppl.DedispPlan(**cfg, dtype=dtype)
+    exp = orc.dedisperse(host, d, p["nout"])
+    assert np.array_equal(plan.run(dev).cpu().numpy(), exp)
+    plan.set_tile(32, 512, 1)
+    assert np.array_equal(plan.run(dev).cpu().numpy(), exp)
+
+
 def test_plan_counts_fused_delay_differences(orc, ppl):
     """The plan reports how many delays a fused multiply-add trial value
     (DedispersionKernel.cu:29 under contraction) would change: none with
