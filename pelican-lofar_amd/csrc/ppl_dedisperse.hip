@@ -1671,6 +1671,16 @@ int device_delays(ppl_dedisp_plan* p)
     return PPL_OK;
 }
 
+// Memory for a table that a plan can do without: null where there is none.
+template <typename T>
+T* spare_memory(size_t bytes)
+{
+    void* d = nullptr;
+    if (hipMalloc(&d, bytes) == hipSuccess) return static_cast<T*>(d);
+    (void)hipGetLastError();  // not an error of a later launch
+    return nullptr;
+}
+
 // The window kernel's shape for a plan's sizes, or -1: rows of whole 16-byte
 // pieces, and 32-trial tiles whose delay spread one of its stages holds.  The
 // widest shape whose tiles keep the 256 CUs busy, else the shortest: one tile
@@ -1697,6 +1707,7 @@ int window_shape(int dtype, int tdms, int nOut, int span, int* staging)
 }
 
 // The window kernel's table, built on the device from the plan's delays.
+// Without memory for it the plan runs its tile.
 int window_table(ppl_dedisp_plan* p)
 {
     const int nChan = (int)p->cfg.nChan, nsamp = (int)p->cfg.nsampBuf, elem = elem_bytes(p->cfg.dtype);
@@ -1709,7 +1720,8 @@ int window_table(ppl_dedisp_plan* p)
         return PPL_OK;
     const int nDMTiles = ((int)p->cfg.tdms + kWinTD - 1) / kWinTD;
     const size_t bytes = win_table_bytes(nDMTiles, nChan);
-    PPL_HIP(hipMalloc(&p->d_win, bytes));
+    p->d_win = spare_memory<int4>(bytes);
+    if (!p->d_win) return PPL_OK;
     const size_t n = bytes / sizeof(int4);
     hipLaunchKernelGGL(kWinShapes[shape].table, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, nullptr, p->d_delayT,
                        nChan, nsamp, p->tdmsPad, nDMTiles, win_whole(staging), p->d_win);
@@ -1738,25 +1750,31 @@ int u8_kernel(ppl_dedisp_plan* p)
     if (total % 16 == 0 && total < (1L << 31) && tile_span(p->delays, tdms, nChan, kU8gTD) <= kU8gSpan) {
         const int nTiles = (tdms + kU8gTD - 1) / kU8gTD, nGroups = (nChan + 3) / 4, capacity = u8g_capacity(nChan);
         PPL_CHECK_ARG((long)nTiles * nGroups < (1L << 31), "u8 group table too large");
-        PPL_HIP(hipMalloc(&p->d_u8g, u8g_table_bytes(nTiles, nChan)));
-        PPL_HIP(hipMemset(p->d_u8g, 0, (size_t)nTiles * sizeof(int32_t)));
-        hipLaunchKernelGGL(u8g_table_kernel, dim3((unsigned)((nTiles * nGroups + 3) / 4)), dim3(256), 0, nullptr,
-                           p->d_delayT, nChan, nsamp, tdms, p->tdmsPad, nTiles, capacity, p->d_u8g);
-        PPL_LAUNCHED();
-        std::vector<int32_t> passes(nTiles);
-        PPL_HIP(hipMemcpy(passes.data(), p->d_u8g, nTiles * sizeof(int32_t), hipMemcpyDeviceToHost));
-        long sum = 0;
-        for (int v : passes) sum += v;
-        if (*std::max_element(passes.begin(), passes.end()) <= capacity && (!ring || sum < 2L * nTiles * nGroups))
-            return PPL_OK;
-        PPL_HIP(hipFree(p->d_u8g));
-        p->d_u8g = nullptr;
+        p->d_u8g = spare_memory<int32_t>(u8g_table_bytes(nTiles, nChan));
+        if (p->d_u8g) {
+            PPL_HIP(hipMemset(p->d_u8g, 0, (size_t)nTiles * sizeof(int32_t)));
+            hipLaunchKernelGGL(u8g_table_kernel, dim3((unsigned)((nTiles * nGroups + 3) / 4)), dim3(256), 0, nullptr,
+                               p->d_delayT, nChan, nsamp, tdms, p->tdmsPad, nTiles, capacity, p->d_u8g);
+            PPL_LAUNCHED();
+            std::vector<int32_t> passes(nTiles);
+            PPL_HIP(hipMemcpy(passes.data(), p->d_u8g, nTiles * sizeof(int32_t), hipMemcpyDeviceToHost));
+            long sum = 0;
+            for (int v : passes) sum += v;
+            if (*std::max_element(passes.begin(), passes.end()) <= capacity && (!ring || sum < 2L * nTiles * nGroups))
+                return PPL_OK;
+            PPL_HIP(hipFree(p->d_u8g));
+            p->d_u8g = nullptr;
+        }
     }
     if (ring) {
-        p->nd = p->nt = p->defNd = p->defNt = 8;
-        p->rw = p->defRw = 16;
         const int32_t* tab = nullptr;
-        return ring_table(p, 32, &tab);  // now, not in a first launch that may be captured
+        // now, not in a first launch that may be captured
+        if (ring_table(p, 32, &tab) == PPL_OK) {
+            p->nd = p->nt = p->defNd = p->defNt = 8;
+            p->rw = p->defRw = 16;
+        } else {
+            (void)hipGetLastError();  // no memory: the one-word tile
+        }
     }
     return PPL_OK;
 }
