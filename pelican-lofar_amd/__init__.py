@@ -1248,16 +1248,35 @@ class MultiBeam:
         instead of every instantiated shape.  One tile for the whole batch,
         or with per_beam each beam's own fastest tile (one launch per group
         of beams sharing a tile) when that is faster on the whole batch.
+        (0, 0, 0) is no tile, each beam under the kernel its sizes call for;
+        it is tried whether or not tiles were set or tuned before.
         Returns the tuned dedispersion time per step in ms."""
         import torch
         ins = [bf.tensor() for bf in self.bufs]
-        tile, ms = autotune_batch(self.plans, ins, self.outs, reps=reps, candidates=candidates)
+        old = [p.tile if p.own_tile else None for p in self.plans]
+        for p in self.plans:
+            p.clear_tile()
+
+        def restore():
+            for p, t in zip(self.plans, old):
+                if t is None:
+                    p.clear_tile()
+                else:
+                    p.set_tile(*t)
+
+        try:
+            tile, ms = autotune_batch(self.plans, ins, self.outs, reps=reps, candidates=candidates)
+        except PPLError:
+            restore()
+            raise
         self.tile = tile
+        if tile[:2] == (0, 0):  # the beams run so only without tiles of their own
+            old = [None] * len(old)
         if not per_beam:
+            restore()
             return ms
         # per-beam tiles (each tuned alone), kept only if the grouped launches
         # beat the single batch tile on the whole batch
-        old = [p.tile if p.own_tile else None for p in self.plans]
         for p, x, o in zip(self.plans, ins, self.outs):
             t, _ = autotune_batch([p], [x], [o], reps=reps, candidates=candidates)
             p.set_tile(*t)
@@ -1272,11 +1291,7 @@ class MultiBeam:
         if own_ms < ms:
             self.tile = "own"
             return own_ms
-        for p, t in zip(self.plans, old):
-            if t is None:
-                p.clear_tile()
-            else:
-                p.set_tile(*t)
+        restore()
         return ms
 
     def chunk_lengths(self, b, n_spec):

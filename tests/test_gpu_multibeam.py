@@ -71,6 +71,18 @@ def test_multibeam_equals_single_beam_chains(ppl, dtype, dft):
             assert torch.equal(mb.outs[b], ch.out), ("graph", k, b)
 
 
+def test_multibeam_autotune_finds_the_way_back_from_a_tile(ppl):
+    """No tile is among what a batch with tiles of its own is tuned over; a
+    batch that is left with another tile keeps its beams' own."""
+    mb = ppl.MultiBeam(_specs(ppl, "f32"), max_chunk_samples=1 << 15)
+    for p in mb.plans:
+        p.set_tile(16, 512, 4)
+    mb.autotune(candidates=[(8, 512, 8)])
+    assert mb.tile == (8, 512, 8, 4) and [p.kernel()[:3] for p in mb.plans] == [("one_word", 16, 512)] * 3
+    mb.autotune(candidates=[(0, 0, 0)])
+    assert mb.tile == (0, 0, 0, 4) and [p.kernel()[0] for p in mb.plans] == ["window"] * 3
+
+
 @pytest.mark.parametrize("per_beam", [False, True])
 def test_multibeam_autotune_keeps_results(ppl, per_beam):
     specs = _specs(ppl, "f32")
