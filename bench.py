@@ -422,7 +422,8 @@ def main():
             log("mixed-precision chain " + mdt)
             mc = make_chain(mdt)
             if mdt == "f32":
-                mc.plan.set_tile(*chain.plan.tile)
+                if chain.plan.own_tile:
+                    mc.plan.set_tile(*chain.plan.tile)
                 m_tune = None
             else:
                 m_tune = mc.autotune()
@@ -582,8 +583,6 @@ def precision(args, torch, ppl):
     bp = beam_bandpass(coeffs, N_SUB, n_ch, INTEG, FCH1, foff, SIGMA)
     inv_scale = 127.0 / 10.0
     chains = [("fp32", "f32"), ("bf16x3", "f16"), ("fp16x2", "f16"), ("bf16x3", "u8")]
-    # f32: autotuned; f16 and u8: the tiles the autotuner picks on the LOFAR beam (the u8 ring kernel)
-    tiles = {"f32": None, "f16": (32, 512, 4), "u8": (32, 512, 0, 16)}
     # channeliser error on a sample: 2 subbands x 96 blocks against FP64
     rng = np.random.default_rng(77)
     sample = np.clip(np.rint(rng.normal(0, SIGMA, size=(2, 2, 96 * n_ch, 2))), -32768, 32767).astype(np.int16)
@@ -619,8 +618,8 @@ def precision(args, torch, ppl):
     for dft, dd in chains:
         log("precision: chain dft=%s dedisp=%s" % (dft, dd))
         ch = ppl.BeamChain(N_SUB, n_ch, N_TAPS, coeffs, INTEG, bp, NSAMP_BUF, TDMS, 0.0, DM_STEP, tsamp, FCH1, foff,
-                           dtype=dd, inv_scale=inv_scale, tile=tiles[dd], dft=dft)
-        if tiles[dd] is None:
+                           dtype=dd, inv_scale=inv_scale, dft=dft)
+        if dd == "f32":  # the others run the kernels their sizes call for
             ch.autotune()
         ch.prime(prime)
         for _ in range(args.warmup):
