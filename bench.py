@@ -143,17 +143,37 @@ def gen_chunk(torch, ppl_coeffs, n_samp, sample0, seed, pulses, rfi, impulses=Tr
     return out
 
 
-def traffic_from_profile(dtype):
-    """HBM bytes per dedispersion launch from the committed counter summary
-    (FETCH_SIZE and WRITE_SIZE per dispatch, scaled by a copy of known size),
-    or None when the summary is absent."""
+KERNEL_NAMES = {("window", "f32"): "dedisperse_window_kernel", ("window", "f16"): "dedisperse_window_kernel",
+                ("u8_group", "u8"): "dedisperse_u8_group_kernel", ("ring", "f32"): "dedisperse_ring_kernel",
+                ("ring", "u8"): "dedisperse_u8_ring_kernel", ("one_word", "f32"): "dedisperse_kernel",
+                ("one_word", "f16"): "dedisperse_f16_kernel", ("one_word", "u8"): "dedisperse_u8_kernel"}
+# what bounds a kernel on the LOFAR beam, from the counters of its profile
+KERNEL_NOTES = {
+    "dedisperse_window_kernel": "a lane reads the samples of four trials once into registers, so the adds' own issue "
+                                "binds (one per clock and lane)",
+    "dedisperse_ring_kernel": "one address add per eight adds (72 VALU instructions per 64 adds); 0.64 VALU "
+                              "wave-instructions per CU-clock against the 1.19 the channeliser sustains, so LDS binds: "
+                              "the 16-byte reads and the staging of four shifted copies of every row"}
+
+
+def dedisp_kernel(plan, d_in, dtype):
+    """The dedispersion kernel that ran on d_in, with its tile."""
+    name, tile_dm, tile_t, staging = plan.kernel(d_in)
+    return {"name": KERNEL_NAMES[name, dtype], "tile_dm": tile_dm, "tile_t": tile_t, "staging": staging,
+            "set_tile_dm_t_chanblock_readbytes": list(plan.tile) if plan.own_tile else None}
+
+
+def traffic_from_profile(dtype, kernel):
+    """HBM bytes per launch of a dedispersion kernel from the committed counter
+    summary (FETCH_SIZE and WRITE_SIZE per dispatch, scaled by a copy of known
+    size), or None where it has no line for that kernel."""
     path = os.path.join(ROOT, "profiles", "dedisperse_lofar_beam_counters.md")
     try:
         with open(path) as f:
             for ln in f:
                 w = ln.split()
-                if len(w) == 3 and w[0] == "traffic_bytes_per_launch" and w[1] == dtype:
-                    return float(w[2])
+                if len(w) == 4 and w[:3] == ["traffic_bytes_per_launch", dtype, kernel]:
+                    return float(w[3])
     except OSError:
         pass
     return None
@@ -388,20 +408,16 @@ def main():
     alg_bytes = N_CHAN * NSAMP_BUF * elem + TDMS * nout * 4
     t_dd = stages["dedisperse"] * 1e-3
     achieved = adds / t_dd / 1e12
-    kname = {"f32": "dedisperse_kernel", "f16": "dedisperse_f16_kernel", "u8": "dedisperse_u8_kernel"}[dd_dtype]
-    if dd_dtype == "f32" and chain.plan.tile[3] == 16:
-        kname = "dedisperse_ring_kernel"
+    dd_kernel = dedisp_kernel(chain.plan, chain.buf.tensor(), dd_dtype)
+    kname = dd_kernel["name"]
     roofline = {"bound": "valu", "achieved": round(achieved, 3), "peak": PEAK_TFLOPS_FP32, "unit": "TFLOP/s",
-                "frac": round(achieved / PEAK_TFLOPS_FP32, 4), "traffic": traffic_from_profile(dd_dtype),
+                "frac": round(achieved / PEAK_TFLOPS_FP32, 4), "traffic": traffic_from_profile(dd_dtype, kname),
                 "traffic_source": "profiles/dedisperse_lofar_beam_counters.md (rocprofv3 --pmc FETCH_SIZE, "
                                   "WRITE_SIZE per dispatch, scaled by a copy of known size; not measured in this run)",
                 "kernel": kname, "ops_per_launch": adds, "alg_bytes_per_launch": alg_bytes,
                 "hbm_gbs_algorithmic": round(alg_bytes / t_dd / 1e9, 1),
-                "note": "ops are channel-order FP32 adds (no FMA, no packed FP32), priced against the FP32 peak: "
-                        "one v_add_f32 per add plus one address add per eight (72 VALU instructions per 64 "
-                        "adds); counters show 0.64 VALU wave-instructions per CU-clock against the 1.19 the "
-                        "channeliser sustains, so LDS binds: the 16-byte reads plus the LDS-DMA staging of "
-                        "four shifted copies of every row (a variant staging one copy ran 17 % faster)"}
+                "note": "ops are channel-order adds (no FMA, no packed FP32), priced against the FP32 peak"
+                        + ("; " + KERNEL_NOTES[kname] if kname in KERNEL_NOTES else "")}
 
     # ---- mixed precision: the same inputs through chains with FP16 / u8
     # dedispersion input (FP32 / int32 sums), against a plain FP32 chain.
@@ -437,7 +453,7 @@ def main():
             mwall = time.perf_counter() - t0
             rec = {"value": TDMS * nout * args.steps / mwall, "ms_per_step": 1e3 * mwall / args.steps,
                    "dedisperse_ms": round(sum(ev[3].elapsed_time(ev[4]) for ev in mt) / args.steps, 3),
-                   "tile_dm_t_chanblock_readbytes": list(mc.plan.tile),
+                   "dedisp_kernel": dedisp_kernel(mc.plan, mc.buf.tensor(), mdt),
                    "autotune_ms": None if m_tune is None else round(m_tune, 3),
                    "events": sum(len(e[0]) - 1 for e in mev)}
             # one more step by hand, keeping the dedispersion input: its series
@@ -520,7 +536,7 @@ def main():
         "config": {"workload": "lofar-beam: 62 sub x 2 pol x 64 ch (3968 ch), 8-tap PPF, Stokes-I x4, "
                                "RFI clipper, 2048 DMs 0-500 on 65536-sample buffers, 6-sigma detection",
                    "nOut_per_step": nout, "input_samples_per_stream_per_step": n_samp,
-                   "dedisp_input": dd_dtype, "dft": "fp32", "tile_dm_t_chanblock_readbytes": list(chain.plan.tile),
+                   "dedisp_input": dd_dtype, "dft": "fp32", "dedisp_kernel": dd_kernel,
                    "autotune_ms": None if tune_ms is None else round(tune_ms, 3)},
         "real_time_factor": rtf,
         "schedule": schedule,
@@ -649,7 +665,7 @@ def precision(args, torch, ppl):
         del keep
         series = (ch.series if dd == "u8" else ch.out).double()
         e64 = (series[fp64[0]] - fp64[1]).abs()
-        rec = {"dft": dft, "dedisp_input": dd, "tile_dm_t_chanblock_readbytes": list(ch.plan.tile),
+        rec = {"dft": dft, "dedisp_input": dd, "dedisp_kernel": dedisp_kernel(ch.plan, ch.buf.tensor(), dd),
                "ms_per_step": round(1e3 * wall, 3),
                "value": TDMS * nout / wall, "real_time_factor": nout * tsamp / wall, "stages_ms": stages,
                "events": sum(len(e) - 1 for e in events),
@@ -774,7 +790,8 @@ def multibeam(args, torch, ppl):
                "graph_value": mb.trials_samples() / gwall,
                "real_time_factor_aggregate": sum(secs) / wall, "real_time_factor_min_beam": min(secs) / wall,
                "stages_ms": stages,
-               "tile_dm_t_chanblock_readbytes": list(mb.tile) if mb.tile != "own" else [list(p.tile) for p in mb.plans],
+               "tile_dm_t_chanblock_readbytes": list(mb.tile) if mb.tile != "own" else
+               [list(p.tile) if p.own_tile else None for p in mb.plans],
                "dft": "fp32" if dtype == "f32" else "bf16x3 (64, 256 ch), fp32 (16 ch)",
                "autotune_ms": round(tune_ms, 3),
                "autotune_s": round(tune_s, 1), "resident_gb": round(mem_gb, 1), "warmup_steps": warm,
