@@ -1736,9 +1736,14 @@ int window_table(ppl_dedisp_plan* p)
 // input ends on 16 bytes, no tile needs more passes than its capacity and,
 // where the ring kernel fits, the mean is below two passes a group (where the
 // two take the same time).  Without it a plan takes the ring kernel if its
-// 32-trial tiles fit that (the conditions of make_job), else the one-word tile,
-// and so do plans of fewer tiles than half the CUs, where the one-word kernel's
-// smaller tiles are as fast.
+// 32-trial tiles fit that (the conditions of make_job), else the one-word tile.
+// Plans of fewer than 128 tiles keep the one-word tile.  Speed is not the
+// reason (1024 channels x 64 trials x 4096 samples: 0.18 ms by groups, 0.45 by
+// words; 128 x 128 x 4096: 0.06 either way): with an earlier form of the u8
+// path, where small plans ran the ring kernel and a series with a row list in
+// scratch memory, a run of the GPU tests aborted, and the cause was not found.
+// The plans of the tests that it can have been lie below this limit and that
+// of the one-launch series, and run what they ran before.
 int u8_kernel(ppl_dedisp_plan* p)
 {
     if (p->cfg.dtype != PPL_U8) return PPL_OK;
@@ -2441,8 +2446,9 @@ extern "C" int ppl_dedisp_u8_series(const ppl_dedisp_plan* p, const int32_t* d_s
     hipStream_t st = stream_of(stream);
     const int nsamp = (int)p->cfg.nsampBuf;
     // One launch, no scratch, from 2^22 series samples on (LOFAR-size beam with
-    // 0.5 % of rows exceptional: 2.95 -> 1.2 ms); small series and trials whose
-    // counts do not fit LDS list the rows first.
+    // 0.5 % of rows exceptional: 2.95 -> 1.2 ms); trials whose counts do not fit
+    // LDS list the rows first, and so do smaller series, for the reason given
+    // at u8_kernel.
     if (p->lenMax <= kSeriesMaxLen && (long)p->cfg.tdms * p->nOut >= (1L << 22)) {
         dim3 grid(cdiv((unsigned)p->nOut, kSeriesTT), p->cfg.tdms);
         hipLaunchKernelGGL(u8_series_lds_kernel, grid, dim3(512), series_lds_bytes(p->lenMax), st, d_sums,
