@@ -280,7 +280,8 @@ enum {
 // In 52640 spectra of a LOFAR beam 242 are such, with 2 to 16 open channels
 // each: a pass of the workgroup over the whole spectrum took 8.3 us and ended
 // a speculative block, 173 spectra long on average; with them in the blocks
-// (511 long) the walk takes 2.85 ms instead of 6.0.
+// (511 long) the walk takes 2.85 ms instead of 6.0, and 2.2 with its present
+// folds.
 constexpr int kUndMax = 16;
 struct UndRec {
     int n;        // undecided channels
@@ -1406,8 +1407,9 @@ __global__ __launch_bounds__(kWalkThreads) void clip_walk_kernel(BatchIO io, int
         // next sixteen before the adds of these, and run past the end to a
         // whole sixteen (the arrays have that room, what is written there is
         // not read, and the result is read back from the last spectrum).
-        // 511 spectra: 6.2 us a fold, 27 cycles a spectrum with its two adds;
-        // with waits for LDS and a select per spectrum for an offset that
+        // 511 spectra: 6.2 us a fold, 27 cycles a spectrum with its two adds
+        // (which take 10 by themselves, measured as a chain in one lane); with
+        // waits for LDS and a select per spectrum for an offset that
         // does not move it was 6.5 and 9.8.
         constexpr int B = kStagePad;
         auto ld16 = [](float* r, const float* a, int k) {
