@@ -2640,6 +2640,7 @@ static int prepare(ppl_clipper* c, const ppl_clip_job& j)
         c->d_und = nullptr;
         c->d_learn = nullptr;
         c->d_stats = nullptr;
+        c->recCap = 0;  // should one of these fail, the next run makes them all
         PPL_HIP(hipMalloc(&c->d_rec, sizeof(SpecRec) * j.nT));
         PPL_HIP(hipMalloc(&c->d_pre, sizeof(PreRec) * j.nT));     // a split run precomputes the whole run
         PPL_HIP(hipMalloc(&c->d_und, sizeof(UndRec) * j.nT));

@@ -20,6 +20,7 @@ void set_error(const char* fmt, ...);
         if (e_ != hipSuccess) {                                                        \
             ::ppl::set_error("%s:%d %s: %s", __FILE__, __LINE__, #expr,                \
                              hipGetErrorString(e_));                                   \
+            (void)hipGetLastError(); /* returned here, not by a later launch check */  \
             return PPL_E_HIP;                                                          \
         }                                                                              \
     } while (0)

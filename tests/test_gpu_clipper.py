@@ -179,6 +179,27 @@ def test_split_run_equals_run(orc, ppl):
     b.run_back()
 
 
+def test_run_after_a_refused_one(orc, ppl):
+    """A run of more spectra than the card has memory for records of is
+    refused; the next one makes its records anew and gives the oracle's
+    outputs, flags and statistics."""
+    n_sub, n_ch = 8, 16
+    x = _stream(3000, n_sub, n_ch, seed=81)
+    bp = _bp(n_sub, n_ch)
+    oc = orc.Clipper(bp, 10.0, 4.0, 1000, True)
+    gc = ppl.Clipper(bp, 10.0, 4.0, 1000, True)
+    for chunk in (x[:2000], x[2000:]):
+        ref = np.ascontiguousarray(chunk)
+        d = torch.from_numpy(ref.copy()).cuda()
+        oc.run(ref)
+        if chunk.shape[0] < 2000:
+            n_max = (1 << 31) - 1  # 136 bytes each: more than the card holds
+            assert ppl.lib().ppl_clipper_run(gc.h, d.data_ptr(), None, n_max, n_sub, 1, n_ch, None) != 0
+        gc.run(d)
+        assert np.array_equal(gc.flags(chunk.shape[0]), oc.last_flags(chunk.shape[0])[0])
+        assert np.array_equal(d.cpu().numpy(), ref, equal_nan=True)
+
+
 @pytest.mark.parametrize("n_und,every", [(2, 40), (16, 40), (17, 40), (5, 9)])
 def test_clipper_rejected_with_undecided_channels(orc, ppl, n_und, every):
     """Every 40th (9th) spectrum loses half its channels to interference, so
